@@ -1399,8 +1399,12 @@ __device__ __forceinline__ void qgemm_body(GemmBatch batch, const Code16 &code) 
   // Every iteration issues the loads of block kb+LOOK; past the last block the
   // last block is loaded again (valid addresses, into the stage that is free)
   // so that the loop body has no branches and schedules as one region.
+  // The counted waits below rely on the loads being issued block by block: nothing of block 1 may move ahead of
+  // block 0's x loads (with few x loads per block the compiler hoisted block 1's codes over them, and the
+  // first wait left block 0's tile in flight).
   WR w0, w1, w2;
   issue(0, 0, w0);
+  asm volatile("" ::: "memory");
   if constexpr (STAGES == 3) {
     issue(1, min(1, nblk - 1), w1);
     wait_vmcnt<LPB>();
@@ -1694,12 +1698,15 @@ __device__ __forceinline__ void qgemm_body(GemmBatch batch, const Code16 &code) 
   }
 }
 
+// Waves per SIMD a tile leaves room for: the accumulators of CB = 1 tiles of at most 192 rows fit twice.
+constexpr int gemm_occupancy(int MB, int CB) { return MB * CB <= 6 ? 2 : 1; }
+
 template <int MB, int CB, int STAGES, int NW, bool SPLIT = false>
-__global__ __launch_bounds__(64 * NW, 1) void nf4_gemm_kernel(GemmBatch batch, Code16 code) {
+__global__ __launch_bounds__(64 * NW, gemm_occupancy(MB, CB)) void nf4_gemm_kernel(GemmBatch batch, Code16 code) {
   qgemm_body<WCodec::kNF4, MB, CB, STAGES, NW, SPLIT>(batch, code);
 }
 template <int MB, int CB, int STAGES, int NW, bool SPLIT = false>
-__global__ __launch_bounds__(64 * NW, 1) void int8_row_gemm_kernel(GemmBatch batch) {
+__global__ __launch_bounds__(64 * NW, gemm_occupancy(MB, CB)) void int8_row_gemm_kernel(GemmBatch batch) {
   qgemm_body<WCodec::kInt8Row, MB, CB, STAGES, NW, SPLIT>(batch, Code16{});
 }
 
@@ -1762,11 +1769,11 @@ __global__ __launch_bounds__(256) void gemm_tail_sum(GemmBatch batch) {
 // fp32 partial tiles of a split launch: split * tail tiles of 256 x 256 floats.
 constexpr int64_t kSplitTileBytes = 256 * 256 * 4;
 
-// How a tiled batch runs: tile height 32 * mb, and whether the last round's
-// `tail` tiles run as `split` K ranges each. Chosen from the shapes and the
-// GPU's CU count only, so a call's bits never depend on anything else.
+// How a tiled batch runs: tiles of 32 * mb rows and 128 * cb columns, and whether
+// the last round's `tail` tiles run as `split` K ranges each. Chosen from the
+// shapes and the GPU's CU count only, so a call's bits never depend on anything else.
 struct GemmPlan {
-  int mb = 8;
+  int mb = 8, cb = 2;
   int split = 1;
   int64_t tail = 0;
   int64_t workspace_bytes() const { return split > 1 ? tail * split * kSplitTileBytes : 0; }
@@ -1786,9 +1793,9 @@ void launch_gemm(GemmBatch &batch, const Code16 &c, hipStream_t s, WCodec wc, in
     tiles += tiles_m * tiles_n;
   }
   constexpr int64_t kTileBytes = 32 * MB * 32 * CB * NW * 4;
-  static_assert(MB != 8 || kTileBytes == kSplitTileBytes, "split tile size");
+  static_assert(MB != 8 || CB != 2 || kTileBytes == kSplitTileBytes, "split tile size");
   batch.tiles = static_cast<int>(tiles);
-  batch.tail = MB == 8 && split > 1 ? static_cast<int>(tiles % cu_count()) : 0;
+  batch.tail = MB == 8 && CB == 2 && split > 1 ? static_cast<int>(tiles % cu_count()) : 0;
   batch.split = batch.tail ? split : 1;
   batch.part = batch.tail ? part : nullptr;
   batch.per_xcd = static_cast<int>(cdiv(tiles - batch.tail, 8));
@@ -1798,7 +1805,7 @@ void launch_gemm(GemmBatch &batch, const Code16 &c, hipStream_t s, WCodec wc, in
   if (batch.tail == 0) {
     if (wc == WCodec::kInt8Row) int8_row_gemm_kernel<MB, CB, STAGES, NW><<<grid, block, 0, s>>>(batch);
     else nf4_gemm_kernel<MB, CB, STAGES, NW><<<grid, block, 0, s>>>(batch, c);
-  } else if constexpr (MB == 8) {
+  } else if constexpr (MB == 8 && CB == 2) {
     if (wc == WCodec::kInt8Row) int8_row_gemm_kernel<MB, CB, STAGES, NW, true><<<grid, block, 0, s>>>(batch);
     else nf4_gemm_kernel<MB, CB, STAGES, NW, true><<<grid, block, 0, s>>>(batch, c);
     const int64_t groups = static_cast<int64_t>(batch.tail) * (kTileBytes / 16);
@@ -1816,7 +1823,8 @@ void launch_gemm(GemmBatch &batch, const Code16 &c, hipStream_t s, WCodec wc, in
 // N 3072) takes 252 224-row ones, the same single round.
 // 128 x 512 tiles of 8 waves (128 x 64 each, two waves per SIMD) measured 15-25 %
 // slower: each decoded weight fragment then serves 4 MFMAs instead of 8.
-GemmPlan plan_gemm(const GemmBatch &batch, WCodec wc) {
+// Launches whose tiles leave CUs idle take narrower tiles (plan_gemm below).
+GemmPlan plan_wide_tiles(const GemmBatch &batch, WCodec wc) {
   auto cost = [&](int mb, double tile_time) {
     int64_t tiles = 0;
     for (int i = 0; i < batch.count; ++i) tiles += cdiv(batch.p[i].M, 32 * mb) * cdiv(batch.p[i].N, 256);
@@ -1869,7 +1877,66 @@ GemmPlan plan_gemm(const GemmBatch &batch, WCodec wc) {
   return plan;
 }
 
+// Tiles of 256, 192 or 128 rows x 128 columns (CB = 1) beside the 256-column ones:
+// their launch has twice to four times the tiles, which pays where 256-column tiles
+// leave CUs idle. Every output still sums K in the same order, so the bits do not
+// change. Decode work per MFMA doubles at least, so a full GPU runs them slower: the
+// estimate of a tile is the larger of its own time on an idle GPU (f us + c us per
+// K block) and its share of what the full GPU sustains (r TFLOP/s), round by round.
+// f, c from K = 3072 and 15360 at M 768, N 3072; r from M 4608, N 21504, K 3072
+// (measured, NF4):
+//   tile       f    c      r          tile       f    c      r
+//   256x256   7.4  1.12  1180         256x128   4.8  0.68   990
+//   224x256   7.3  1.02  1130         192x128   4.4  0.60   990
+//   192x256   6.6  0.94  1080         128x128   4.1  0.53   860
+// Examples (us, before -> now): 768 x 3072 x 3072 52 -> 29, 768 x 3072 x 12288
+// 184 -> 102, 1536 x 3072 x 15360 237 -> 176, 768 x 9216 x 3072 58 -> 48.
+// The narrow tile has to win by 4 % (the estimates' error at full rounds).
+struct TileCost {
+  int mb, cb;
+  double f, c, r;
+};
+constexpr TileCost kWideCost[] = {{8, 2, 7.4, 1.12, 1180e6}, {7, 2, 7.3, 1.02, 1130e6}, {6, 2, 6.6, 0.94, 1080e6}};
+constexpr TileCost kNarrowCost[] = {{8, 1, 4.8, 0.68, 990e6}, {6, 1, 4.4, 0.60, 990e6}, {4, 1, 4.1, 0.53, 860e6}};
+
+// Estimated us of a launch of whole tiles.
+double tile_estimate(const GemmBatch &batch, const TileCost &t) {
+  int64_t tiles = 0;
+  int kmax = 0;
+  for (int i = 0; i < batch.count; ++i) {
+    tiles += cdiv(batch.p[i].M, 32 * t.mb) * cdiv(batch.p[i].N, 128 * t.cb);
+    kmax = std::max(kmax, batch.p[i].K);
+  }
+  const double alone = t.f + t.c * (kmax / 64), flops = 2.0 * (32 * t.mb) * (128 * t.cb) * kmax;
+  const int64_t cu = cu_count(), full = tiles / cu, rest = tiles % cu;
+  auto round = [&](int64_t n) { return n == 0 ? 0.0 : std::max(alone, t.f + n * flops / t.r); };
+  return full * round(cu) + round(rest);
+}
+
+GemmPlan plan_gemm(const GemmBatch &batch, WCodec wc) {
+  GemmPlan plan = plan_wide_tiles(batch, wc);
+  if (plan.split > 1) return plan;
+  double best = 0.96 * tile_estimate(batch, kWideCost[8 - plan.mb]);
+  for (const TileCost &t : kNarrowCost) {
+    const double e = tile_estimate(batch, t);
+    if (e < best) {
+      best = e;
+      plan.mb = t.mb;
+      plan.cb = t.cb;
+    }
+  }
+  return plan;
+}
+
 void launch_plan(GemmBatch &batch, const GemmPlan &plan, const Code16 &c, hipStream_t s, WCodec wc, float *part) {
+  if (plan.cb == 1) {
+    switch (plan.mb) {
+      case 4: launch_gemm<4, 1, 3, 4>(batch, c, s, wc, 1, nullptr); break;
+      case 6: launch_gemm<6, 1, 3, 4>(batch, c, s, wc, 1, nullptr); break;
+      default: launch_gemm<8, 1, 3, 4>(batch, c, s, wc, 1, nullptr); break;
+    }
+    return;
+  }
   switch (plan.mb) {
     case 6: launch_gemm<6, 2, 3, 4>(batch, c, s, wc, 1, nullptr); break;
     case 7: launch_gemm<7, 2, 3, 4>(batch, c, s, wc, 1, nullptr); break;
