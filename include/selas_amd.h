@@ -81,6 +81,15 @@ int selas_nf4_encode(const float *w, int64_t n, int64_t blocksize, const float c
                      float *absmax, void *stream);
 
 /*
+ * selas_nf4_encode of a tensor of dtype w_dtype (the exact conversion to fp32
+ * is part of the kernel). 16-bit tensors need blocksize 64, 16-byte alignment
+ * and a codebook in [-1, 1] whose midpoints ascend at least 1/16 apart
+ * (otherwise SELAS_EUNSUPPORTED: convert to fp32 first).
+ */
+int selas_nf4_encode_typed(const void *w, int w_dtype, int64_t n, int64_t blocksize, const float code[16],
+                           uint8_t *packed, float *absmax, void *stream);
+
+/*
  * int8_row decode of a weight of `rows` rows of `cols` elements (q int8
  * [rows, cols], scale fp32 [rows]):
  *   out[r, c] = dtype(float(q[r, c]) * float(dtype(scale[r])))
@@ -98,6 +107,14 @@ int selas_int8_row_dequant(const int8_t *q, const float *scale, int64_t rows, in
  * Replaces encode_int8_row (selas/codecs.py:86-96).
  */
 int selas_int8_row_encode(const float *w, int64_t rows, int64_t cols, int8_t *q, float *scale, void *stream);
+
+/*
+ * selas_int8_row_encode of a weight of dtype w_dtype (the exact conversion to
+ * fp32 is part of the kernel). 16-bit weights need 16-byte alignment and cols a
+ * multiple of 8, at most 16384 (otherwise SELAS_EUNSUPPORTED: convert first).
+ */
+int selas_int8_row_encode_typed(const void *w, int w_dtype, int64_t rows, int64_t cols, int8_t *q, float *scale,
+                                void *stream);
 
 /* ------------------------------------------------------------ linear */
 

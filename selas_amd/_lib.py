@@ -28,6 +28,7 @@ _F16x = ctypes.POINTER(ctypes.c_float)
 SIGNATURES: dict[str, list] = {
     "selas_nf4_dequant": [_P, _P, _I64, _I64, _F16x, _P, _INT, _P],
     "selas_nf4_encode": [_P, _I64, _I64, _F16x, _P, _P, _P],
+    "selas_nf4_encode_typed": [_P, _INT, _I64, _I64, _F16x, _P, _P, _P],
     "selas_nf4_linear": [_P, _I64, _I64, _I64, _P, _P, _I64, _F16x, _I64, _P, _P, _I64, _INT, _P, _I64, _P],
     "selas_nf4_linear_grouped": [_P, _I64, _I64, _I64, _P, _I64, _I64, _I64, _F16x, _INT, _P],
     "selas_nf4_linear_batched": [_P, _I64, _I64, _F16x, _INT, _P, _I64, _P],
@@ -35,6 +36,7 @@ SIGNATURES: dict[str, list] = {
     "selas_nf4_linear_grouped_static": [_P, _I64, _I64, _I64, _P, _I64, _I64, _F16x, _INT, _P],
     "selas_int8_row_dequant": [_P, _P, _I64, _I64, _P, _INT, _P],
     "selas_int8_row_encode": [_P, _I64, _I64, _P, _P, _P],
+    "selas_int8_row_encode_typed": [_P, _INT, _I64, _I64, _P, _P, _P],
     "selas_int8_row_linear": [_P, _I64, _I64, _I64, _P, _P, _I64, _P, _P, _I64, _INT, _P, _I64, _P],
     "selas_int8_row_linear_batched": [_P, _I64, _INT, _P, _I64, _P],
     "selas_int8_row_linear_grouped": [_P, _I64, _I64, _I64, _P, _I64, _I64, _INT, _P],

@@ -59,6 +59,19 @@ def _gpu_for(t: torch.Tensor) -> torch.device:
     return torch.device("cuda", torch.cuda.current_device())
 
 
+def _float_on(t: torch.Tensor, dev: torch.device) -> torch.Tensor:
+    """t on ``dev`` in a dtype the encoders read: its own when that is fp32, bf16 or fp16, else fp32."""
+    return t.detach().to(device=dev, dtype=t.dtype if t.dtype in _lib.DTYPE_CODES else torch.float32)
+
+
+def _encode_typed(launch, w: torch.Tensor) -> None:
+    """``launch(w)``, and where the encoder does not take w's 16-bit form, ``launch`` of its fp32 copy."""
+    try:
+        launch(w)
+    except _lib.Unsupported:
+        launch(w.float())
+
+
 def encode_nf4(name: str, t: torch.Tensor, blocksize: int = 64, code: tuple[float, ...] = NF4_CODE) -> EncodedTensor:
     """NF4-encodes ``t`` (selas/codecs.py:99-119) with the GPU encoder.
 
@@ -70,12 +83,16 @@ def encode_nf4(name: str, t: torch.Tensor, blocksize: int = 64, code: tuple[floa
     if blocksize <= 0 or n % blocksize or blocksize % 2:
         raise ValueError(f"nf4 needs numel divisible by blocksize ({n} % {blocksize}) for {name}")
     dev = _gpu_for(t)
-    flat = t.detach().to(device=dev, dtype=torch.float32).reshape(-1).contiguous()
+    flat = _float_on(t, dev).reshape(-1).contiguous()
     packed = torch.empty(n // 2, dtype=torch.uint8, device=dev)
     absmax = torch.empty(n // blocksize, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        _lib.call("selas_nf4_encode", flat.data_ptr(), n, blocksize, _lib.code_array(code), packed.data_ptr(),
-                  absmax.data_ptr(), _lib.stream(dev))
+
+    def launch(w):
+        with torch.cuda.device(dev):
+            _lib.call("selas_nf4_encode_typed", w.data_ptr(), _lib.dtype_code(w.dtype), n, blocksize,
+                      _lib.code_array(code), packed.data_ptr(), absmax.data_ptr(), _lib.stream(dev))
+
+    _encode_typed(launch, flat)
     if t.device.type != "cuda":
         packed, absmax = packed.cpu(), absmax.cpu()
     return EncodedTensor(name, "nf4", tuple(t.shape), {"blocksize": blocksize, "code": list(code)},
@@ -145,11 +162,16 @@ def encode_int8_row(name: str, t: torch.Tensor) -> EncodedTensor:
     dev = _gpu_for(t)
     rows = int(t.shape[0])
     cols = t.numel() // rows if rows else 0
-    w = t.detach().to(device=dev, dtype=torch.float32).reshape(rows, cols).contiguous()
+    flat = _float_on(t, dev).reshape(rows, cols).contiguous()
     q = torch.empty(tuple(t.shape), dtype=torch.int8, device=dev)
     scale = torch.empty(rows, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        _lib.call("selas_int8_row_encode", w.data_ptr(), rows, cols, q.data_ptr(), scale.data_ptr(), _lib.stream(dev))
+
+    def launch(w):
+        with torch.cuda.device(dev):
+            _lib.call("selas_int8_row_encode_typed", w.data_ptr(), _lib.dtype_code(w.dtype), rows, cols, q.data_ptr(),
+                      scale.data_ptr(), _lib.stream(dev))
+
+    _encode_typed(launch, flat)
     if t.device.type != "cuda":
         q, scale = q.cpu(), scale.cpu()
     return EncodedTensor(name, "int8_row", tuple(t.shape), {}, {"q": q, "scale": scale})

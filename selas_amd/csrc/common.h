@@ -26,6 +26,20 @@ inline const char *dtype_name(int dt) {
   return dt == SELAS_F32 ? "f32" : dt == SELAS_F16 ? "f16" : dt == SELAS_BF16 ? "bf16" : "?";
 }
 
+// Division of 31-bit indices by a fixed d >= 1: i / d = (i * mul) >> shift exactly, since mul * d exceeds 2^shift by
+// less than d <= 2^(shift - 31).
+struct FastDiv {
+  uint32_t mul, shift;
+};
+inline FastDiv fast_div(uint32_t d) {
+  uint32_t s = 0;
+  while ((1ull << s) < d) ++s;
+  return FastDiv{static_cast<uint32_t>(((1ull << (31 + s)) + d - 1) / d), 31 + s};
+}
+__host__ __device__ inline uint32_t div31(uint32_t i, FastDiv f) {
+  return static_cast<uint32_t>((static_cast<uint64_t>(i) * f.mul) >> f.shift);
+}
+
 // The 16-entry codebook, passed by value so that it lives in scalar registers.
 struct Code16 {
   float v[16];
@@ -145,6 +159,36 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 // GELU of two values rounded as a packed bf16 pair (the hardware convert).
 __device__ __forceinline__ uint32_t gelu_bf16x2(float lo, float hi) {
   return pack_bf16x2(gelu_tanh_fast(lo), gelu_tanh_fast(hi));
+}
+
+// Eight consecutive 16-bit or fp32 elements as fp32, and the largest |w| bits among them: magnitude bits order like
+// the values, with NaN above Inf, so an unsigned maximum is the NaN-propagating one.
+template <int DT>
+__device__ __forceinline__ uint32_t load8(const void *p, int64_t i8, float (&v)[8]) {
+  uint32_t m = 0;
+  if constexpr (DT == SELAS_F32) {
+    const uint4 *s = static_cast<const uint4 *>(p) + 2 * i8;
+    const uint4 u0 = s[0], u1 = s[1];
+    const uint32_t w[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+#pragma unroll
+    for (int t = 0; t < 8; ++t) v[t] = __uint_as_float(w[t]);
+  } else {
+    const uint4 u = static_cast<const uint4 *>(p)[i8];
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      if constexpr (DT == SELAS_BF16) {
+        v[2 * t] = __uint_as_float(w[t] << 16);
+        v[2 * t + 1] = __uint_as_float(w[t] & 0xffff0000u);
+      } else {
+        v[2 * t] = f16_bits_to_f32(w[t] & 0xffffu);
+        v[2 * t + 1] = f16_bits_to_f32(w[t] >> 16);
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 8; ++t) m = max(m, __float_as_uint(v[t]) & 0x7fffffffu);
+  return m;
 }
 
 // Wave-wide (64 lanes) reductions through the cross-lane network.
