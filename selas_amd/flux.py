@@ -25,7 +25,7 @@ import torch.nn.functional as F
 
 from .codecs import EncodedTensor, encode_int8_row, encode_nf4, encode_raw
 from .kernels import FUSED, Kernels
-from .linear import UnitView, int8_row_linear_grouped, nf4_linear_grouped
+from .linear import UnitView, linear_grouped_into
 
 
 @dataclass
@@ -344,24 +344,31 @@ class RandomFlux:
         ``grouped`` runs all modulation linears in one launch (same bits as one call per linear)."""
         pre = self.mod_prefixes()
         codecs = {u.tensors[p + ".weight"].codec for u, p in pre}
-        if grouped and codecs == {"nf4"}:
-            ws = []
-            for u, p in pre:
-                e = u.tensors[p + ".weight"]
-                ws.append((e.parts["packed"], e.parts["absmax"], int(e.meta["blocksize"]), e.meta["code"], e.shape,
-                           u.get(p + ".bias")))
-            ys = nf4_linear_grouped(sv, ws)
-        elif grouped and codecs == {"int8_row"}:
-            ws = []
-            for u, p in pre:
-                e = u.tensors[p + ".weight"]
-                ws.append((e.parts["q"], e.parts["scale"], e.shape, u.get(p + ".bias")))
-            ys = int8_row_linear_grouped(sv, ws)
-        else:
-            ys = [u.linear(sv, p) for u, p in pre]
+        nd = len(self.doubles)
+        if grouped and len(codecs) == 1 and codecs <= {"nf4", "int8_row"}:
+            # Each double block's image and text vectors are written side by side, where the block reads them: a
+            # concatenation of the two afterwards took 5.8 us per double block (110 us beside the launch's 408).
+            codec = codecs.pop()
+            ws, out, per = [], [], []
+            for j, u in enumerate(self.mods):
+                ps = ("img_mod.lin", "txt_mod.lin") if j < nd else ("modulation.lin",)
+                width = 0
+                for p in ps:
+                    e = u.tensors[p + ".weight"]
+                    width += e.shape[0]
+                    if codec == "nf4":
+                        ws.append((e.parts["packed"], e.parts["absmax"], int(e.meta["blocksize"]), e.meta["code"],
+                                   e.shape, u.get(p + ".bias")))
+                    else:
+                        ws.append((e.parts["q"], e.parts["scale"], None, None, e.shape, u.get(p + ".bias")))
+                out.append(torch.empty(*sv.shape[:-1], width, dtype=sv.dtype, device=sv.device))
+                per.append(len(ps))
+            linear_grouped_into(codec, sv, ws, out, per)
+            return out
+        ys = [u.linear(sv, p) for u, p in pre]
         out, i = [], 0
         for j in range(len(self.mods)):
-            if j < len(self.doubles):
+            if j < nd:
                 out.append(torch.cat((ys[i], ys[i + 1]), dim=-1))
                 i += 2
             else:

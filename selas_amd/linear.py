@@ -318,11 +318,12 @@ class GroupedPlan:
     table and the outputs are built once; ``run(x)`` is one kernel launch and returns the
     plan's own output tensors, which the next ``run`` overwrites. ``supported`` is False
     when the grouped kernel does not cover the shapes (then ``nf4_linear_grouped`` runs the
-    linears one by one).
+    linears one by one). ``dst``: optional (address, row stride) per weight for the plan to write
+    instead of outputs of its own (``outs`` is then empty and the caller keeps the memory).
     """
 
     def __init__(self, weights, rows: int, device: torch.device, dtype: torch.dtype = torch.bfloat16,
-                 codec: str = "nf4"):
+                 codec: str = "nf4", dst: list[tuple[int, int]] | None = None):
         self.codec = codec
         self.weights = list(weights)
         self.rows = int(rows)
@@ -333,27 +334,30 @@ class GroupedPlan:
         self.desc = None
         if not self.supported:
             return
-        rows_tbl, total_n = [], 0
-        for packed, absmax, bs, _, shape, bias in self.weights:
+        table, total_n = [], 0
+        for i, (packed, absmax, bs, _, shape, bias) in enumerate(self.weights):
             n = int(shape[0])
             _check_parts(codec, packed, absmax, n, self.k, 64 if bs is None else bs)
             if bias is not None and (bias.dtype != dtype or not bias.is_contiguous()):
                 bias = bias.to(dtype).contiguous()
                 self._keep.append(bias)
             _check_bias(bias, n)
-            y = torch.empty(self.rows, n, dtype=dtype, device=device)
-            self.outs.append(y)
-            rows_tbl.append([packed.data_ptr(), absmax.data_ptr(), 0 if bias is None else bias.data_ptr(),
-                             y.data_ptr(), n, n])
+            if dst is None:
+                y = torch.empty(self.rows, n, dtype=dtype, device=device)
+                self.outs.append(y)
+                to = (y.data_ptr(), n)
+            else:
+                to = dst[i]
+            table += (packed.data_ptr(), absmax.data_ptr(), 0 if bias is None else bias.data_ptr(), to[0], n, to[1])
             total_n += n
         self.total_n = total_n
-        self.desc = torch.tensor(rows_tbl, dtype=torch.int64).to(device)
+        self.desc = torch.tensor(table, dtype=torch.int64).view(-1, 6).to(device)
         self.code = _lib.code_array(self.weights[0][3]) if codec == "nf4" else None
 
     def _eligible(self, dtype) -> bool:
         if self.codec == "nf4":
-            codes = {tuple(float(c) for c in w[3]) for w in self.weights}
-            if len(codes) != 1 or any(int(w[2]) != 64 for w in self.weights):
+            code = self.weights[0][3]
+            if any(w[3] is not code and tuple(w[3]) != tuple(code) or int(w[2]) != 64 for w in self.weights):
                 return False
         return (dtype == torch.bfloat16 and 1 <= self.rows <= GROUPED_MAX_M and self.k in GROUPED_K
                 and len(self.weights) <= GROUPED_MAX_WEIGHTS
@@ -391,6 +395,35 @@ def nf4_linear_grouped(x: torch.Tensor, weights) -> list[torch.Tensor]:
     return _grouped("nf4", x, list(weights))
 
 
+def linear_grouped_into(codec: str, x: torch.Tensor, weights, bufs: list[torch.Tensor], per: list[int]) -> None:
+    """``nf4_linear_grouped`` (or ``int8_row_linear_grouped``; ``weights`` as GroupedPlan's) with the results of the
+    first per[0] weights side by side in the columns of bufs[0], those of the next per[1] in bufs[1], and so on.
+    Each buffer is contiguous, [..., sum n_i] in x's dtype and device with x's leading dims."""
+    weights = list(weights)
+    rows = x.numel() // x.shape[-1]
+    dst, i = [], 0
+    for buf, count in zip(bufs, per):
+        at, ld, size = buf.data_ptr(), buf.shape[-1], buf.element_size()
+        for w in weights[i:i + count]:
+            dst.append((at, ld))
+            at += int(w[4][0]) * size
+        i += count
+    dev = _lib.require_gpu(x, *(w[0] for w in weights))
+    x2 = _rows(x)
+    plan = GroupedPlan(weights, rows, dev, x.dtype, codec, dst)
+    if _plan_takes(plan, x2):
+        plan.run(x2)
+        return
+    i = 0
+    for buf, count in zip(bufs, per):
+        torch.cat([_single(codec, (x, *w)) for w in weights[i:i + count]], dim=-1, out=buf)
+        i += count
+
+
+def _plan_takes(plan: GroupedPlan, x2: torch.Tensor) -> bool:
+    return plan.supported and x2.data_ptr() % 16 == 0 and x2.stride(0) % 8 == 0 and x2.shape[1] == plan.k
+
+
 def int8_row_linear_grouped(x: torch.Tensor, weights) -> list[torch.Tensor]:
     """``nf4_linear_grouped`` for int8_row weights: (q, scale, shape, bias) tuples sharing ``x``."""
     return _grouped("int8_row", x, [(q, s, None, None, shape, b) for q, s, shape, b in weights])
@@ -402,7 +435,7 @@ def _grouped(codec: str, x: torch.Tensor, weights) -> list[torch.Tensor]:
     dev = _lib.require_gpu(x, *(w[0] for w in weights))
     x2 = _rows(x)
     plan = GroupedPlan(weights, x2.shape[0], dev, x.dtype, codec)
-    if not plan.supported or x2.data_ptr() % 16 or x2.stride(0) % 8 or x2.shape[1] != plan.k:
+    if not _plan_takes(plan, x2):
         return [_single(codec, (x, *w)) for w in weights]
     outs = plan.run(x2)
     # The plan's descriptor table may be freed now: the caching allocator hands its memory

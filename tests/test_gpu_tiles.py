@@ -59,3 +59,17 @@ def test_narrow_tiles(codec, m, n, k):
         gelu = nf4_linear_gelu if codec == "nf4" else int8_row_linear_gelu
         ((plain, g),) = gelu([(x, *args, b, 256, None)])
         assert torch.equal(plain, y[:, :n - 256]) and torch.equal(g, Kernels().gelu(y[:, n - 256:]))
+
+
+@pytest.mark.parametrize("quant", ["nf4", "int8"])
+@pytest.mark.parametrize("rows", [1, 5, 33])
+def test_modulations_side_by_side(quant, rows):
+    # The grouped launch writes a double block's image and text vectors into one buffer: the bits of the linears one by
+    # one and their concatenation; 33 rows are past the grouped kernel.
+    from selas_amd import flux as F
+
+    cfg = F.FluxConfig(hidden=1024, heads=8, mlp_hidden=512)
+    m = F.RandomFlux(cfg, "cuda", seed=3, n_double=2, n_single=3, quant=quant)
+    sv = torch.randn(rows, 1, cfg.hidden, generator=seeded(rows)).to(torch.bfloat16).cuda()
+    one, got = m.modulations(sv, grouped=False), m.modulations(sv)
+    assert len(got) == 5 and all(a.shape == b.shape and torch.equal(a, b) for a, b in zip(one, got))
