@@ -386,6 +386,14 @@ int selas_attention(const void *q, const void *k, const void *vt, int64_t B, int
                     void *out, int64_t ldo, int dtype, void *stream);
 
 /*
+ * selas_attention with the values as v [B, H, L, Dh] in place of v^T: the
+ * kernel transposes them on their way to the matrix cores. Same bits. At most
+ * 65535 heads.
+ */
+int selas_attention_v(const void *q, const void *k, const void *v, int64_t B, int64_t H, int64_t L, int64_t Dh,
+                      void *out, int64_t ldo, int dtype, void *stream);
+
+/*
  * vt[i, d, l] = v[i, l, d] for BH heads of [L, Dh] (bf16, Dh = 128), with vt rows
  * of Lp = L rounded up to a multiple of 64 tokens and vt[i, d, l] = 0 for l >= L:
  * the value layout selas_attention reads. No counterpart in the reference.

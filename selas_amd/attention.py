@@ -3,9 +3,9 @@
 The reference calls ``F.scaled_dot_product_attention(q, k, v)`` on q, k, v
 [B, H, L, Dh] and returns ``out.transpose(1, 2).reshape(B, L, H * Dh)``.
 ``attention`` computes the same with one fused kernel that writes the
-[B, L, H * Dh] layout directly (the transpose copy disappears). The values are
-read transposed ([B, H, Dh, L] padded to a multiple of 64 tokens), produced by
-``transpose_heads``. Any sequence length runs; shapes outside the kernel (head
+[B, L, H * Dh] layout directly (the transpose copy disappears) and reads v as it
+is. ``transpose_heads`` lays v out as the C entry ``selas_attention`` takes it.
+Any sequence length runs; shapes outside the kernel (head
 dim other than 128, dtypes other than bf16) raise ``Unsupported``;
 ``flux.attention`` then runs SDPA, as the reference.
 """
@@ -59,8 +59,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tens
           or out.stride(0) != l * out.stride(1)):
         raise ValueError(f"attention: out must be [{b}, {l}, {h * d}] {q.dtype} on {q.device} with unit column "
                          f"stride and equally spaced rows, got {tuple(out.shape)} strides {out.stride()}")
-    vt = transpose_heads(v)
+    v = _heads(v, "attention")
     with torch.cuda.device(dev):
-        _lib.call("selas_attention", q.data_ptr(), k.data_ptr(), vt.data_ptr(), b, h, l, d, out.data_ptr(),
+        _lib.call("selas_attention_v", q.data_ptr(), k.data_ptr(), v.data_ptr(), b, h, l, d, out.data_ptr(),
                   out.stride(1), _lib.dtype_code(q.dtype), _lib.stream(dev))
     return out

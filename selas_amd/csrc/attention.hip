@@ -2,9 +2,9 @@
 // softmax(q k^T / sqrt(128)) v for every (batch, head), written straight into the
 // [B, L, H * 128] layout the projection linear reads.
 //
-// One workgroup = NWV waves (8 when L >= 3072, else 4) = 32 * NWV queries of
+// One workgroup = NWV waves (8 or 4, see the launch) = 32 * NWV queries of
 // one (batch, head); wave w owns queries 32w .. 32w+31. The keys stream through
-// LDS in tiles of 64 (K rows and the matching V^T columns, double-buffered,
+// LDS in tiles of 64 (K rows and the matching V rows, double-buffered,
 // loaded by buffer->LDS DMA, shared by all the workgroup's waves). Per tile:
 //   * S^T = K Q^T on 32x32x16 MFMAs (16 per wave): K from LDS is the A operand,
 //     Q (held in registers for the whole loop) the B operand, so lane l holds 32
@@ -16,12 +16,16 @@
 //     operand straight from the score registers. For that, the K rows of a 32-key
 //     block are loaded with bits 2 and 3 of the row index swapped: lane (q, h)
 //     register r then holds key 16*(r/8) + 8*h + r%8, i.e. 8 consecutive keys per
-//     MFMA k-step, and the V^T operand reads 8 consecutive keys (16 bytes).
+//     MFMA k-step, as the V^T operand holds, transposed by the LDS reads
+//     (ds_read_b64_tr_b16). With v^T laid out by a kernel of its own (16-byte
+//     operand reads) the product itself ran 4 % faster at L = 4608, but that
+//     kernel cost 11 us there and half a call's time at L < 1024: 48.7 -> 42.1 us
+//     for B1 L 1536, 258.5 -> 254.6 us for B1 L 4608.
 // LDS tiles are XOR-swizzled in 16-byte chunks so that the fragment reads (16
 // lanes per LDS cycle) hit 16 distinct 4-bank groups.
 // Any sequence length: key and query rows past L read as zeros (buffer range),
 // the last key tile's missing keys get score -inf, and query rows past L are not
-// stored; v^T rows are padded with zeros to a multiple of 64 tokens.
+// stored; value rows past L read as zeros too (v^T: padded to 64 tokens).
 //
 // LDS bandwidth bounds this kernel: every MFMA reads a 1 KiB A fragment from LDS
 // (halving those reads ran 24 % faster). Two query blocks per wave would share
@@ -29,7 +33,9 @@
 // ran 25 % slower, because a lone wave cannot overlap its softmax with MFMAs.
 // Eight waves per workgroup (one workgroup per CU) share each tile's DMA among
 // 256 queries instead of 128, which cuts the LDS traffic per query by a tenth.
+#include <atomic>
 #include <type_traits>
+
 #include "common.h"
 
 namespace selas {
@@ -65,10 +71,11 @@ __device__ __forceinline__ uint32_t pack_probs(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
-template <int NWV>
+// VT: the values come as v^T [B*H, 128, Lp] (selas_attention), else as v [B*H, L, 128] (selas_attention_v).
+template <int NWV, bool VT>
 __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *__restrict__ q,
                                                                const uint16_t *__restrict__ k,
-                                                               const uint16_t *__restrict__ vt,
+                                                               const uint16_t *__restrict__ v,
                                                                uint16_t *__restrict__ out, int64_t ldo, int H, int L,
                                                                int qtiles, int per_xcd, int total, float c2) {
   constexpr int kQT = 32 * NWV;  // queries per workgroup
@@ -82,15 +89,16 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int h = lane >> 5, c = lane & 31;
-  // q, k: [B*H, L, 128]; v^T: [B*H, 128, Lp] with Lp = L rounded up to the 64-key tile
-  // (zero-filled). Query and key rows past L read as zeros through the buffer range.
+  // q, k, v: [B*H, L, 128]; v^T: [B*H, 128, Lp] with Lp = L rounded up to the 64-key tile
+  // (zero-filled). Query, key and value rows past L read as zeros through the buffer range.
   const int Lp = (L + kKT - 1) / kKT * kKT;
   const int64_t head = static_cast<int64_t>(bh) * L * kDh;  // elements
   const uint32_t head_bytes = static_cast<uint32_t>(L) * kDh * 2;
   const __amdgpu_buffer_rsrc_t qr = make_rsrc(q + head, head_bytes);
   const __amdgpu_buffer_rsrc_t kr = make_rsrc(k + head, head_bytes);
-  const __amdgpu_buffer_rsrc_t vr = make_rsrc(vt + static_cast<int64_t>(bh) * Lp * kDh,
-                                              static_cast<uint32_t>(Lp) * kDh * 2);
+  const __amdgpu_buffer_rsrc_t vr = VT ? make_rsrc(v + static_cast<int64_t>(bh) * Lp * kDh,
+                                                   static_cast<uint32_t>(Lp) * kDh * 2)
+                                       : make_rsrc(v + head, head_bytes);
 
   // Q as the B operand of S^T = K Q^T: lane (query c of this wave, h) holds d = 16s + 8h .. +8.
   const int q_row = qt * kQT + 32 * wave + c;
@@ -99,20 +107,25 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
   for (int s = 0; s < 8; ++s)
     qf[s] = __builtin_bit_cast(bf16x8, load_b128(qr, static_cast<uint32_t>(q_row) * 256u + (16 * s + 8 * h) * 2, 0));
 
-  // DMA per tile: 16 instructions of 1 KiB for K (4 rows of 256 B each) and 16
-  // for V^T (8 rows of 128 B), KJ + KJ per wave. Lane i of K instruction J fills
-  // row r = 4J + i/16, physical chunk i%16, with logical chunk (i%16) ^ (r%16);
-  // lane i of V^T instruction J fills row d = 8J + i/8, physical chunk i%8, with
-  // logical chunk (i%8) ^ ((d/2)%8). The tile's first key goes in the scalar offset.
+  // DMA per tile: 16 instructions of 1 KiB for K and V (4 rows of 256 B each; V^T:
+  // 8 rows of 128 B) each, KJ + KJ per wave. Lane i of instruction J fills row
+  // r = 4J + i/16, physical chunk i%16, with logical chunk (i%16) ^ (r%16) of K,
+  // (i%16) ^ 4(r%4) of V; lane i of V^T instruction J fills row d = 8J + i/8,
+  // physical chunk i%8, with logical chunk (i%8) ^ ((d/2)%8). The tile's first key
+  // goes in the scalar offset.
   uint32_t k_voff[KJ], v_voff[KJ];
 #pragma unroll
   for (int j = 0; j < KJ; ++j) {
     const int J = KJ * wave + j;
     const int r = 4 * J + (lane >> 4);
     k_voff[j] = static_cast<uint32_t>(r) * 256u + ((static_cast<uint32_t>(lane & 15) ^ (r & 15)) << 4);
-    const int d = 8 * J + (lane >> 3);
-    v_voff[j] = static_cast<uint32_t>(d) * static_cast<uint32_t>(Lp) * 2u +
-                ((static_cast<uint32_t>(lane & 7) ^ ((d >> 1) & 7)) << 4);
+    if constexpr (VT) {
+      const int d = 8 * J + (lane >> 3);
+      v_voff[j] = static_cast<uint32_t>(d) * static_cast<uint32_t>(Lp) * 2u +
+                  ((static_cast<uint32_t>(lane & 7) ^ ((d >> 1) & 7)) << 4);
+    } else {
+      v_voff[j] = static_cast<uint32_t>(r) * 256u + ((static_cast<uint32_t>(lane & 15) ^ (4 * (lane >> 4))) << 4);
+    }
   }
   auto issue = [&](int stage, int kt) {
     uint8_t *base = smem + stage * kStageBytes;
@@ -120,7 +133,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
 #pragma unroll
     for (int j = 0; j < KJ; ++j) load_lds16(kr, base + (KJ * wave + j) * 1024, k_voff[j], key0 * 256u);
 #pragma unroll
-    for (int j = 0; j < KJ; ++j) load_lds16(vr, base + kTileBytes + (KJ * wave + j) * 1024, v_voff[j], key0 * 2u);
+    for (int j = 0; j < KJ; ++j) load_lds16(vr, base + kTileBytes + (KJ * wave + j) * 1024, v_voff[j], key0 * (VT ? 2u : 256u));
   };
   // A-operand fragments: K row of MFMA row c in key block kb, d-chunk 2s+h; V^T
   // row d = 32db + c, key chunk 4kb + 2t + h (keys 32kb + 16t + 8h .. +8).
@@ -130,11 +143,31 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
     const int cc = 2 * s + h;
     return *reinterpret_cast<const bf16x8 *>(smem + stage * kStageBytes + r * 256 + ((cc ^ (r & 15)) << 4));
   };
+  // V as the A operand of O^T += V^T P^T: lane (c, h) needs channel 32db + c of the keys 32kb + 16t + 8h .. +8.
+  // ds_read_b64_tr_b16 transposes on the way: the 16 lanes of a group each address 4 channels of one of 4 keys (lane
+  // i: key i/4, channels 4(i%4) .. +4), and lane i receives channel i of the 4 keys. Two reads make an operand. The
+  // swizzle puts the 4 keys of a read in 4 different quarters of the 256-byte rows, so it is free of bank conflicts.
+  uint32_t v_rd[4];
+  {
+    const int r = (lane >> 2) & 3, x = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);
+#pragma unroll
+    for (int db = 0; db < 4; ++db) v_rd[db] = (8 * h + r) * 256 + ((db ^ r) << 6) + x * 16 + 8 * (lane & 1);
+  }
   auto vfrag = [&](int stage, int db, int kb, int t2) {
-    const int d = 32 * db + c;
-    const int cc = 4 * kb + 2 * t2 + h;
-    return *reinterpret_cast<const bf16x8 *>(smem + stage * kStageBytes + kTileBytes + d * 128 +
-                                             ((cc ^ ((d >> 1) & 7)) << 4));
+    uint8_t *vs = smem + stage * kStageBytes + kTileBytes;
+    if constexpr (VT) {
+      const int d = 32 * db + c;
+      const int cc = 4 * kb + 2 * t2 + h;
+      return *reinterpret_cast<const bf16x8 *>(vs + d * 128 + ((cc ^ ((d >> 1) & 7)) << 4));
+    } else {
+      typedef short s16x4 __attribute__((ext_vector_type(4)));
+      auto read = [&](int u) {
+        return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(
+            vs + v_rd[db] + kb * 8192 + t2 * 4096 + u * 1024));
+      };
+      const s16x4 lo = read(0), hi = read(1);
+      return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
   };
 
   f32x16 o[4];
@@ -156,7 +189,10 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
     // Scores: 16 MFMAs over (key block kb, d-chunk s) = (i / 8, i % 8). The K
     // fragments go through a ring of kKAhead registers, each read kKAhead MFMAs
     // before its use, so that no MFMA waits on a read issued just before it.
+    // A wave in its scores goes ahead of the SIMD's other wave (1 % at L = 4608; also
+    // around the output product, or the exponentials ahead, measured slower).
     constexpr int kKAhead = 4;
+    __builtin_amdgcn_s_setprio(1);
     f32x16 sc[2] = {f32x16{}, f32x16{}};
     bf16x8 kf[kKAhead];
 #pragma unroll
@@ -183,6 +219,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
         for (int r = 0; r < 16; ++r)
           if (kt * kKT + 32 * kb + 16 * (r >> 3) + 8 * h + (r & 7) >= L) sc[kb][r] = -__builtin_inff();
     }
+    __builtin_amdgcn_s_setprio(0);
     float mx = sc[0][0];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
@@ -201,7 +238,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
     }
     // V^T fragments of the second product (db, kb, t2) = (i / 4, (i / 2) % 2, i % 2),
     // the first kVAhead read before the exponentials, the rest kVAhead MFMAs ahead.
-    constexpr int kVAhead = 8;
+    constexpr int kVAhead = VT ? 8 : 6;  // two reads a fragment from V: 6 measured 1 % faster than 8, as 4
     bf16x8 vf[kVAhead];
 #pragma unroll
     for (int i = 0; i < kVAhead; ++i) vf[i] = vfrag(stage, i / 4, (i / 2) % 2, i % 2);
@@ -319,30 +356,67 @@ int check_heads(const char *what, int64_t B, int64_t H, int64_t L, int64_t Dh, i
 }
 }  // namespace
 
-extern "C" int selas_attention(const void *q, const void *k, const void *vt, int64_t B, int64_t H, int64_t L,
-                               int64_t Dh, void *out, int64_t ldo, int dtype, void *stream) {
-  if (int e = check_heads("attention", B, H, L, Dh, dtype)) return e;
+namespace {
+// The GPU's CU count (256 on MI355X), asked of the runtime once per device.
+int attn_cu_count() {
+  static std::atomic<int> counts[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
+    (void)hipGetLastError();
+    dev = 0;
+  }
+  int v = counts[dev].load(std::memory_order_relaxed);
+  if (v > 0) return v;
+  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) {
+    (void)hipGetLastError();
+    v = 256;
+  }
+  counts[dev].store(v, std::memory_order_relaxed);
+  return v;
+}
+
+template <bool VT>
+int attention_any(const char *what, const void *q, const void *k, const void *v, int64_t B, int64_t H, int64_t L,
+                  int64_t Dh, void *out, int64_t ldo, int dtype, void *stream) {
+  if (int e = check_heads(what, B, H, L, Dh, dtype)) return e;
   if (B == 0 || H == 0 || L == 0) return ok();
-  if (!q || !k || !vt || !out) return set_error(SELAS_EINVAL, "attention: null pointer");
-  if (ldo < H * Dh) return set_error(SELAS_EINVAL, "attention: out row stride %lld below H*Dh", (long long)ldo);
-  if (!aligned(q, 16) || !aligned(k, 16) || !aligned(vt, 16) || !aligned(out, 8) || ldo % 4)
-    return set_error(SELAS_EUNSUPPORTED, "attention: q, k, v^T must be 16-byte aligned, out rows 8-byte aligned");
+  if (!q || !k || !v || !out) return set_error(SELAS_EINVAL, "%s: null pointer", what);
+  if (ldo < H * Dh) return set_error(SELAS_EINVAL, "%s: out row stride %lld below H*Dh", what, (long long)ldo);
+  if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 8) || ldo % 4)
+    return set_error(SELAS_EUNSUPPORTED, "%s: q, k and the values must be 16-byte aligned, out rows 8-byte aligned", what);
   const float c2 = 1.4426950408889634f / sqrtf(static_cast<float>(Dh));  // log2(e) / sqrt(Dh)
   auto launch = [&](auto kernel, int nwv) {
     const int qtiles = static_cast<int>(cdiv(L, 32 * nwv));
     const int64_t total = B * H * qtiles;
     const int per_xcd = static_cast<int>(cdiv(total, 8));
     kernel<<<dim3(static_cast<uint32_t>(per_xcd * 8)), dim3(64 * nwv), 0, static_cast<hipStream_t>(stream)>>>(
-        static_cast<const uint16_t *>(q), static_cast<const uint16_t *>(k), static_cast<const uint16_t *>(vt),
+        static_cast<const uint16_t *>(q), static_cast<const uint16_t *>(k), static_cast<const uint16_t *>(v),
         static_cast<uint16_t *>(out), ldo, static_cast<int>(H), static_cast<int>(L), qtiles, per_xcd,
         static_cast<int>(total), c2);
   };
-  // Eight waves share each tile among more queries but run one workgroup per CU:
-  // at L = 4608 (FLUX 1024^2) 282 us against 297 with four, at L = 1536 159 against
-  // 151 (each workgroup's fixed costs weigh more over 24 key tiles than over 72).
-  if (L >= 3072) launch(attn_fwd_kernel<8>, 8);
-  else launch(attn_fwd_kernel<4>, 4);
-  return check_launch("attention");
+  // Eight waves share each tile among more queries but run one workgroup per CU; of the four-wave workgroups two
+  // run on a CU, or one, faster, when there are no more than CUs left. Relative time per key tile of a round of each
+  // (us, fitted to B 1 and 4 at L = 768 to 4608 with 24 heads): 1.74, 1.9 and 1.3. Measured, four waves against
+  // eight, us: B1 L 4608 274 / 251, B1 L 1536 45.7 / 42.4, B2 L 2300 145 / 135, B4 L 1536 127 / 142, B1 L 768 18 / 25.
+  const int64_t cu = attn_cu_count(), n8 = B * H * cdiv(L, 256), n4 = B * H * cdiv(L, 128), rest = n4 % (2 * cu);
+  const double t8 = 1.74 * static_cast<double>(cdiv(n8, cu));
+  const double t4 = 1.9 * static_cast<double>(n4 / (2 * cu)) + (rest == 0 ? 0.0 : rest <= cu ? 1.3 : 1.9);
+  if (t8 < t4) launch(attn_fwd_kernel<8, VT>, 8);
+  else launch(attn_fwd_kernel<4, VT>, 4);
+  return check_launch(what);
+}
+}  // namespace
+
+extern "C" int selas_attention(const void *q, const void *k, const void *vt, int64_t B, int64_t H, int64_t L,
+                               int64_t Dh, void *out, int64_t ldo, int dtype, void *stream) {
+  return attention_any<true>("attention", q, k, vt, B, H, L, Dh, out, ldo, dtype, stream);
+}
+
+extern "C" int selas_attention_v(const void *q, const void *k, const void *v, int64_t B, int64_t H, int64_t L,
+                                 int64_t Dh, void *out, int64_t ldo, int dtype, void *stream) {
+  if (B >= 0 && H >= 0 && B * H > 65535)
+    return set_error(SELAS_EUNSUPPORTED, "attention_v: more than 65535 heads");
+  return attention_any<false>("attention_v", q, k, v, B, H, L, Dh, out, ldo, dtype, stream);
 }
 
 extern "C" int selas_transpose_heads(const void *v, int64_t BH, int64_t L, int64_t Dh, void *vt, int dtype,
