@@ -1485,9 +1485,11 @@ __device__ __forceinline__ void qgemm_body(GemmBatch batch, const Code16 &code) 
     // One scheduling region per K block. Without this fence the slot matching
     // of the interleave shifts by one sub-step after the first block's barrier
     // and two thirds of the x-fragment reads land 3-5 MFMAs before their use;
-    // with it most land 9-13 MFMAs ahead (NF4 block linears +1.3 %). The int8 operand's
-    // reads stay about 3 MFMAs ahead with or without it.
-    if constexpr (!kI8) __builtin_amdgcn_sched_barrier(0);
+    // with it most land 9-13 MFMAs ahead (NF4 block linears +1.3 %). For int8 the
+    // scheduler also pulled the next block's byte conversions up to right behind
+    // their loads, which drained every load in flight once or twice per three
+    // blocks: linear1 531 -> 494 us, linear2 400 -> 348 us with the fence.
+    __builtin_amdgcn_sched_barrier(0);
   };
 
   // In the split kernel, wait here for everything read through the scalar cache
