@@ -6,7 +6,7 @@
 //
 // Kernels, chosen from M and K:
 //   * M <= 32 (hoisted adaLN modulation linears, M = number of steps), HBM-bound:
-//     nf4_gemv_stream for K = 1024, 2048, 3072 (one launch can cover many
+//     nf4_gemv_few (M <= 2) and nf4_gemv_stream for K = 1024, 2048, 3072 (one launch can cover many
 //     weights), nf4_gemv_kernel for other K. Both multiply x by the codes on
 //     MFMA and apply the block's fp32 absmax to the fp32 block partial sums;
 //     codes come from bank-replicated LDS tables indexed by the packed byte.
@@ -749,6 +749,180 @@ __global__ __launch_bounds__(64 * NW, 1) void nf4_gemv_stream(
   finish((it - 1) & (L::kRedBufs - 1), d_prev, row_prev, bias_prev);
 }
 
+// ------------------------------------------------------- few-row streaming GEMV
+//
+// For M <= 2 and K = 1024, 2048, 3072, one or many weights (a step's or two steps' modulation linears). HBM-bound, and
+// a single weight is short (32 MB): what counts is the time to the first byte and no work between the loads.
+// nf4_gemv_stream spends 9 us of a launch on x in MFMA order, the first unit's latency and the 8-wave reduction, and
+// gives 576 units of 32 rows to 256 CUs (three rounds for two and a quarter).
+//
+// Here a wave takes whole rows (wave w of W: rows w, w + W, ...), four in flight: a row is 512 bytes of codes per
+// 1024 columns, 8 bytes (16 codes) per lane and load, so loads are coalesced and x stays in registers in the same
+// order. Codes are looked up as in nf4_gemv_stream (a byte gives an fp16 code pair, 64 replicas, one v_perm and one
+// ds_read_b32), v_dot2_f32_f16 multiplies them with x in fp16 (each lane's part of a row of x scaled by a power of
+// two of its own, as there per wave) and the fp32 sum of a lane's 16 codes is scaled by their block's absmax. The
+// lanes' sums are added by a butterfly, always in the same order: the same bits alone and in a group.
+// 18432 x 3072 from Python at M = 1: 13.1 us, where the host's 13 us a call shows (nf4_gemv_stream 14.6), M = 2 14.0
+// (14.6); 76 weights in a launch 400 and 407 us, 4.6 TB/s (417 and 419).
+constexpr int kFewMaxM = 2;  // at M = 4 its work per code passes the matrix cores': 18.3 us against 14.7
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+template <int KC, int MM, int NW>
+__global__ __launch_bounds__(64 * NW, 1) void nf4_gemv_few(const uint16_t *__restrict__ x, int64_t ldx, int M,
+                                                           const GemvDesc *__restrict__ descs, int count, GemvDesc one,
+                                                           Code16 code) {
+  constexpr int kblocks = 16 * KC, row_bytes = 512 * KC, kThreads = 64 * NW;
+  extern __shared__ __align__(16) uint32_t lds_words[];
+  uint8_t *lds = reinterpret_cast<uint8_t *>(lds_words);
+  int *prefix = reinterpret_cast<int *>(lds + kSgTableBytes);  // [g] = rows before weight g
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // x first: its latency covers the table and the prefix. Lane's chunk j of a row: columns 16 (64 j + lane) .. +16.
+  uint4 xr[MM][KC][2];
+#pragma unroll
+  for (int m = 0; m < MM; ++m) {
+    const auto r = make_rsrc(x + static_cast<int64_t>(min(m, M - 1)) * ldx, 2048u * KC);
+#pragma unroll
+    for (int j = 0; j < KC; ++j)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) xr[m][j][t] = load_b128(r, 32u * (64 * j + lane) + 16 * t, 0);
+  }
+  {
+    constexpr int kParts = kThreads / 256, kPer = 64 / kParts;
+    const int b = tid & 255, part = tid >> 8;
+    float hi = 0.0f, lo = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      hi = (b >> 4) == i ? code.v[i] : hi;
+      lo = (b & 15) == i ? code.v[i] : lo;
+    }
+    const uint32_t e = __builtin_bit_cast(uint16_t, static_cast<_Float16>(hi)) |
+                       (static_cast<uint32_t>(__builtin_bit_cast(uint16_t, static_cast<_Float16>(lo))) << 16);
+#pragma unroll
+    for (int j = 0; j < kPer; ++j)
+      *reinterpret_cast<uint32_t *>(lds + b * 256 + (kPer * part + ((j + lane) & (kPer - 1))) * 4) = e;
+  }
+  if (wave == 0) {
+    int carry = 0;
+    for (int base = 0; base < count; base += 64) {
+      const int g = base + lane;
+      int v = g < count ? static_cast<int>(descs ? descs[g].n : one.n) : 0;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int t = __shfl_up(v, off);
+        if (lane >= off) v += t;
+      }
+      if (g < count) prefix[g + 1] = carry + v;
+      carry += __shfl(v, 63);
+    }
+    if (lane == 0) prefix[0] = 0;
+  }
+  f16x2 xh[MM][KC][8];
+  float inv[MM];
+#pragma unroll
+  for (int m = 0; m < MM; ++m) {
+    // |x| as bf16 magnitude bits; the scale 2^k brings the lane's largest into [2^14, 2^15) (1 for 0, Inf and NaN).
+    uint32_t mx = 0;
+#pragma unroll
+    for (int j = 0; j < KC; ++j)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const uint32_t w[4] = {xr[m][j][t].x, xr[m][j][t].y, xr[m][j][t].z, xr[m][j][t].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = max(mx, max((w[i] >> 16) & 0x7fffu, w[i] & 0x7fffu));
+      }
+    const unsigned e = mx >> 7;
+    const int k = (e == 0u || e == 0xffu) ? 0 : 14 - (static_cast<int>(e) - 127);
+    const float sc = __uint_as_float(static_cast<uint32_t>(max(-126, min(127, k)) + 127) << 23);
+    inv[m] = __uint_as_float(static_cast<uint32_t>(max(-126, min(127, -k)) + 127) << 23);
+#pragma unroll
+    for (int j = 0; j < KC; ++j)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const uint32_t w[4] = {xr[m][j][t].x, xr[m][j][t].y, xr[m][j][t].z, xr[m][j][t].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          xh[m][j][4 * t + i] = f16x2{static_cast<_Float16>(__uint_as_float(w[i] << 16) * sc),
+                                      static_cast<_Float16>(__uint_as_float(w[i] & 0xffff0000u) * sc)};
+      }
+  }
+  __syncthreads();  // table and prefix
+  const int rows = prefix[count], W = gridDim.x * NW;
+  const uint32_t tsel = static_cast<uint32_t>(lane) * 4u;
+  // A row in flight: its codes, scales and bias, and where its results go.
+  struct Row {
+    uint2 q[KC];
+    float s[KC];
+    uint32_t bias;
+    uint16_t *y;
+    int ldy, n;
+  };
+  int g = 0;
+  SDesc d = uniform_desc(descs ? descs[0] : one);
+  auto load = [&](int row, Row &r) __attribute__((always_inline)) {
+    if (row >= rows) return;  // uniform over the wave; compute() skips it too
+    if (prefix[g + 1] <= row) {
+      while (prefix[g + 1] <= row) ++g;
+      g = __builtin_amdgcn_readfirstlane(g);
+      d = uniform_desc(descs ? descs[g] : one);
+    }
+    const int n = __builtin_amdgcn_readfirstlane(row - prefix[g]);
+    const auto rq = make_rsrc(d.packed + static_cast<int64_t>(n) * row_bytes, row_bytes);
+    const auto rs = make_rsrc(d.absmax + static_cast<int64_t>(n) * kblocks, 4 * kblocks);
+#pragma unroll
+    for (int j = 0; j < KC; ++j) {
+      r.q[j] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rq, 8u * lane, 512 * j, 0));
+      r.s[j] = load_f32(rs, 4u * (lane >> 2), 64 * j);
+    }
+    r.bias = 0;
+    if (d.bias) r.bias = __builtin_amdgcn_raw_buffer_load_b16(make_rsrc(d.bias, static_cast<uint32_t>(d.n) * 2u), 0, 2 * n, 0);
+    r.y = d.y;
+    r.ldy = d.ldy;
+    r.n = n;
+  };
+  auto compute = [&](int row, const Row &r) __attribute__((always_inline)) {
+    if (row >= rows) return;
+    float acc[MM] = {};
+#pragma unroll
+    for (int j = 0; j < KC; ++j) {
+      float p[MM] = {};
+      const uint32_t w[2] = {r.q[j].x, r.q[j].y};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        // The table starts at LDS address 0: this kernel declares no static LDS.
+        const uint32_t at = perm(w[i >> 2], tsel, 0x0C0C0400u | ((4u + (i & 3)) << 8));
+        const f16x2 c = __builtin_bit_cast(
+            f16x2, *reinterpret_cast<const __attribute__((address_space(3))) uint32_t *>(static_cast<uintptr_t>(at)));
+#pragma unroll
+        for (int m = 0; m < MM; ++m) p[m] = __builtin_amdgcn_fdot2(c, xh[m][j][i], p[m], false);
+      }
+#pragma unroll
+      for (int m = 0; m < MM; ++m) acc[m] += p[m] * r.s[j];
+    }
+    float v = 0.0f;
+#pragma unroll
+    for (int m = 0; m < MM; ++m) {
+      const float t = wave_sum(acc[m] * inv[m]);
+      v = lane == m ? t : v;
+    }
+    if (lane < M) {
+      const auto ry = make_rsrc(r.y, static_cast<uint32_t>(((M - 1) * r.ldy + r.n + 1) * 2));
+      __builtin_amdgcn_raw_buffer_store_b16(bf16_bits_rne(v + bf16_bits_to_f32(r.bias)), ry,
+                                            static_cast<uint32_t>(lane * r.ldy + r.n) * 2u, 0, 0);
+    }
+  };
+  Row buf[4];
+  int row = blockIdx.x * NW + wave;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) load(row + i * W, buf[i]);
+  for (; row < rows; row += 4 * W) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      compute(row + i * W, buf[i]);
+      load(row + (4 + i) * W, buf[i]);
+    }
+  }
+}
+
 // ------------------------------------------------------- int8_row streaming skinny GEMM
 //
 // For M <= 32, K = 1024, 2048, 3072 and int8_row weights: the structure of
@@ -997,10 +1171,37 @@ int launch_stream(const uint16_t *x, int64_t ldx, int64_t M, const GemvDesc *des
   return check_launch("nf4_linear (streaming skinny gemm)");
 }
 
+template <int KC, int MM>
+int launch_few(const uint16_t *x, int64_t ldx, int64_t M, const GemvDesc *descs, int count, const GemvDesc &one,
+               int64_t total_n, const Code16 &c, hipStream_t s) {
+  constexpr int NW = 16;  // four waves per SIMD; x takes 8 KC MM of the 128 registers each
+  constexpr int kMaxBytes = kSgTableBytes + (kSgMaxDescs + 1) * 4;
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&nf4_gemv_few<KC, MM, NW>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kMaxBytes);
+  if (attr != hipSuccess)
+    return set_error(SELAS_EHIP, "nf4_linear: cannot reserve %d bytes of LDS: %s", kMaxBytes, hipGetErrorString(attr));
+  const int64_t grid = min(cdiv(total_n, NW), static_cast<int64_t>(cu_count()));
+  const size_t lds = kSgTableBytes + (count + 1) * sizeof(int);
+  nf4_gemv_few<KC, MM, NW><<<dim3(static_cast<uint32_t>(grid)), dim3(64 * NW), lds, s>>>(
+      x, ldx, static_cast<int>(M), descs, count, one, c);
+  return check_launch("nf4_linear (few-row gemv)");
+}
+
 // total_n: sum of the weights' row counts (an upper bound on the work, for the grid size).
 int launch_gemv_stream(const uint16_t *x, int64_t ldx, int64_t M, int64_t K, const GemvDesc *descs, int count,
                        const GemvDesc &one, int64_t total_n, const Code16 &c, hipStream_t s) {
   constexpr int NW = kSgWaves;
+  if (M <= kFewMaxM && total_n < (1ll << 30)) {
+#define SELAS_FEW(KC)                                                                    \
+  return M == 1 ? launch_few<KC, 1>(x, ldx, M, descs, count, one, total_n, c, s)          \
+                : launch_few<KC, 2>(x, ldx, M, descs, count, one, total_n, c, s)
+    switch (K) {
+      case 1024: SELAS_FEW(1);
+      case 2048: SELAS_FEW(2);
+      case 3072: SELAS_FEW(3);
+    }
+#undef SELAS_FEW
+  }
   switch (K) {
     case 1024: return launch_stream<NW, 1024 / 64 / NW>(x, ldx, M, descs, count, one, total_n, c, s);
     case 2048: return launch_stream<NW, 2048 / 64 / NW>(x, ldx, M, descs, count, one, total_n, c, s);
@@ -1838,7 +2039,7 @@ GemmPlan plan_wide_tiles(const GemmBatch &batch, WCodec wc) {
   // is then power-bound, shorter tiles in one round finish no sooner, and the
   // taller tile does the same work with fewer tiles (4608 x 3072 x 15360: 374 us
   // with 256-row tiles, 390 us with 224, 574 us with 192). The int8 operand's
-  // kernel keeps the cost model (256-row tiles made that shape slower).
+  // kernel keeps the cost model (256-row tiles: 364 us on that shape, 224-row 348).
   int64_t t8 = 0;
   for (int i = 0; i < batch.count; ++i) t8 += cdiv(batch.p[i].M, 256) * cdiv(batch.p[i].N, 256);
   const int64_t cu = cu_count();
