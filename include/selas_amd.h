@@ -10,7 +10,8 @@
  *     buffer reuse stays correct) and never synchronises the device;
  *   - allocates nothing and frees nothing: outputs and scratch memory are
  *     caller-owned (a tiled linear whose launch splits its last round of tiles
- *     over K takes a workspace argument, sized by selas_linear_workspace_bytes);
+ *     over K takes a workspace argument, sized by selas_linear_workspace_bytes,
+ *     and selas_attention_split one sized by selas_attention_workspace_bytes);
  *   - returns SELAS_OK or an error code and never throws; the message of the
  *     last error on the calling thread is returned by selas_last_error().
  *
@@ -392,6 +393,19 @@ int selas_attention(const void *q, const void *k, const void *vt, int64_t B, int
  */
 int selas_attention_v(const void *q, const void *k, const void *v, int64_t B, int64_t H, int64_t L, int64_t Dh,
                       void *out, int64_t ldo, int dtype, void *stream);
+
+/*
+ * selas_attention_v where a last round of few 256-query items leaves most CUs
+ * idle: those items run as ranges of keys on the idle CUs, their fp32 partial
+ * outputs are kept in `workspace` (device memory, 16-byte aligned, at least
+ * selas_attention_workspace_bytes) and added in key order. The choice and the
+ * size depend on B, H, L and the CU count only; with a size of 0 the call is
+ * selas_attention_v, bit for bit. A workspace that is missing or too small is
+ * SELAS_EINVAL, with nothing launched.
+ */
+int selas_attention_split(const void *q, const void *k, const void *v, int64_t B, int64_t H, int64_t L, int64_t Dh,
+                          void *out, int64_t ldo, int dtype, void *workspace, int64_t workspace_bytes, void *stream);
+int selas_attention_workspace_bytes(int64_t B, int64_t H, int64_t L, int64_t *bytes);
 
 /*
  * vt[i, d, l] = v[i, l, d] for BH heads of [L, Dh] (bf16, Dh = 128), with vt rows

@@ -51,6 +51,8 @@ SIGNATURES: dict[str, list] = {
     "selas_attn_mlp": [_P, _I64, _I64, _I64, _P, _I64, _I64, _P, _INT, _P],
     "selas_attention": [_P, _P, _P, _I64, _I64, _I64, _I64, _P, _I64, _INT, _P],
     "selas_attention_v": [_P, _P, _P, _I64, _I64, _I64, _I64, _P, _I64, _INT, _P],
+    "selas_attention_split": [_P, _P, _P, _I64, _I64, _I64, _I64, _P, _I64, _INT, _P, _I64, _P],
+    "selas_attention_workspace_bytes": [_I64, _I64, _I64, ctypes.POINTER(ctypes.c_int64)],
     "selas_transpose_heads": [_P, _I64, _I64, _I64, _P, _INT, _P],
 }
 

@@ -4,13 +4,16 @@ The reference calls ``F.scaled_dot_product_attention(q, k, v)`` on q, k, v
 [B, H, L, Dh] and returns ``out.transpose(1, 2).reshape(B, L, H * Dh)``.
 ``attention`` computes the same with one fused kernel that writes the
 [B, L, H * Dh] layout directly (the transpose copy disappears) and reads v as it
-is. ``transpose_heads`` lays v out as the C entry ``selas_attention`` takes it.
-Any sequence length runs; shapes outside the kernel (head
+is. Where the last round of workgroups is a small one it is split over the keys,
+by B, H, L and the CU count only. ``transpose_heads`` lays v out as the C entry
+``selas_attention`` takes it. Any sequence length runs; shapes outside the kernel (head
 dim other than 128, dtypes other than bf16) raise ``Unsupported``;
 ``flux.attention`` then runs SDPA, as the reference.
 """
 
 from __future__ import annotations
+
+import ctypes
 
 import torch
 
@@ -60,7 +63,12 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tens
         raise ValueError(f"attention: out must be [{b}, {l}, {h * d}] {q.dtype} on {q.device} with unit column "
                          f"stride and equally spaced rows, got {tuple(out.shape)} strides {out.stride()}")
     v = _heads(v, "attention")
+    size = ctypes.c_int64()
     with torch.cuda.device(dev):
-        _lib.call("selas_attention_v", q.data_ptr(), k.data_ptr(), v.data_ptr(), b, h, l, d, out.data_ptr(),
-                  out.stride(1), _lib.dtype_code(q.dtype), _lib.stream(dev))
+        # 0 unless a last round of few workgroups is split over the keys; on the caller's stream, from torch's pool.
+        _lib.call("selas_attention_workspace_bytes", b, h, l, ctypes.byref(size))
+        n = size.value
+        ws = torch.empty(n, dtype=torch.uint8, device=dev) if n else None
+        _lib.call("selas_attention_split", q.data_ptr(), k.data_ptr(), v.data_ptr(), b, h, l, d, out.data_ptr(),
+                  out.stride(1), _lib.dtype_code(q.dtype), ws.data_ptr() if n else None, n, _lib.stream(dev))
     return out

@@ -71,19 +71,39 @@ __device__ __forceinline__ uint32_t pack_probs(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
+// Items from `whole` on run as `parts` ranges of `per` key tiles each (selas_attention_split); a range leaves each
+// wave's output, not yet divided, and its queries' maxima and sums in `partial`.
+struct AttnSplit {
+  int whole, parts, per;
+  float *partial;
+};
+// Per wave and range: 64 x 64 outputs in the order of the registers (1 KiB per store instruction), then per lane the
+// running maximum and the sum.
+constexpr int kPartialFloats = 64 * 64 + 2 * 64;
+
 // VT: the values come as v^T [B*H, 128, Lp] (selas_attention), else as v [B*H, L, 128] (selas_attention_v).
-template <int NWV, bool VT>
+template <int NWV, bool VT, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *__restrict__ q,
                                                                const uint16_t *__restrict__ k,
                                                                const uint16_t *__restrict__ v,
                                                                uint16_t *__restrict__ out, int64_t ldo, int H, int L,
-                                                               int qtiles, int per_xcd, int total, float c2) {
+                                                               int qtiles, int per_xcd, int total, float c2,
+                                                               AttnSplit sp) {
   constexpr int kQT = 32 * NWV;  // queries per workgroup
   constexpr int KJ = 16 / NWV;   // DMA instructions per wave and tile, for K and for V^T each
   __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * kStageBytes];
   // Work item t = (b % 8) * per_xcd + b / 8: each XCD takes a contiguous range,
   // so the query tiles of one head share that head's K and V^T in its L2.
-  const int t = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  // Split: the whole items first, then the ranges, a range's parts on different XCDs.
+  int t = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3), range = -1;
+  if constexpr (SPLIT) {
+    if (static_cast<int>(blockIdx.x) >= 8 * per_xcd) {
+      range = blockIdx.x - 8 * per_xcd;
+      t = sp.whole + range / sp.parts;
+    } else if (t >= sp.whole) {
+      return;
+    }
+  }
   if (t >= total) return;
   const int bh = t / qtiles, qt = t - bh * qtiles;
   const int tid = threadIdx.x;
@@ -173,10 +193,17 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
   f32x16 o[4];
 #pragma unroll
   for (int db = 0; db < 4; ++db) o[db] = f32x16{};
-  float m_run = -__builtin_inff(), l_run = 0.0f;
-  const int ntiles = Lp / kKT;
+  // Split: a range may hold only scores of -inf, which then weigh nothing beside the other ranges.
+  float m_run = SPLIT ? -3.402823466e38f : -__builtin_inff(), l_run = 0.0f;
+  int kt = 0, ntiles = Lp / kKT;
+  if constexpr (SPLIT) {
+    if (range >= 0) {
+      kt = range % sp.parts * sp.per;
+      ntiles = min(ntiles, kt + sp.per);
+    }
+  }
 
-  issue(0, 0);
+  issue(0, kt);
   wait_vmcnt<0>();
   __syncthreads();
 
@@ -272,19 +299,30 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
   };
   const std::integral_constant<bool, false> full{};
   const std::integral_constant<bool, true> last{};
-  const int nfull = L / kKT;  // tiles whose 64 keys all exist
-  int kt = 0;
+  const int kt0 = kt, nfull = SPLIT ? min(L / kKT, ntiles) : L / kKT;  // tiles whose 64 keys all exist
   for (; kt + 2 <= nfull; kt += 2) {
     tile(0, kt, full);
     tile(1, kt + 1, full);
   }
   if (kt < nfull) tile(0, kt++, full);
-  if (kt < ntiles) {  // a partial last tile, stage kt % 2
-    if (kt & 1) tile(1, kt, last);
+  if (kt < ntiles) {  // a partial last tile
+    if ((kt - kt0) & 1) tile(1, kt, last);
     else tile(0, kt, last);
   }
 
   // out[(b*L + q) * ldo + hh*128 + d] = O^T[d][q] / l, d = 32db + 8g + 4h + e for register 4g + e.
+  if constexpr (SPLIT) {
+    if (range >= 0) {
+      float *w = sp.partial + static_cast<int64_t>(range * NWV + wave) * kPartialFloats;
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        *reinterpret_cast<float4 *>(w + (i * 64 + lane) * 4) =
+            make_float4(o[i >> 2][4 * (i & 3)], o[i >> 2][4 * (i & 3) + 1], o[i >> 2][4 * (i & 3) + 2],
+                        o[i >> 2][4 * (i & 3) + 3]);
+      *reinterpret_cast<float2 *>(w + 4096 + 2 * lane) = make_float2(m_run, pair_sum(l_run));
+      return;
+    }
+  }
   const float inv = 1.0f / pair_sum(l_run);
   const int b = bh / H, hh = bh - b * H;
   if (q_row >= L) return;  // a last query tile past the sequence end
@@ -297,6 +335,44 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
       *reinterpret_cast<uint2 *>(orow + d) = make_uint2(pack_bf16x2(o[db][4 * g] * inv, o[db][4 * g + 1] * inv),
                                                         pack_bf16x2(o[db][4 * g + 2] * inv, o[db][4 * g + 3] * inv));
     }
+}
+
+// The split items' outputs from their ranges, added in key order: a workgroup of one wave per 32 queries and 32
+// channels, in the lane order of attn_fwd_kernel. Bounded by the reads of the partial outputs (L2, Infinity Cache).
+__global__ __launch_bounds__(64) void attn_merge_kernel(const float *__restrict__ partial, uint16_t *__restrict__ out,
+                                                        int64_t ldo, int H, int L, int qtiles, int nwv, int whole,
+                                                        int parts) {
+  const int lane = threadIdx.x, db = blockIdx.x & 3, wave = (blockIdx.x >> 2) % nwv, item = (blockIdx.x >> 2) / nwv;
+  const int t = whole + item, bh = t / qtiles, qt = t - bh * qtiles;
+  const int64_t step = static_cast<int64_t>(nwv) * kPartialFloats;  // from one range to the next
+  const float *w = partial + (static_cast<int64_t>(item) * parts * nwv + wave) * kPartialFloats;
+  float m = -__builtin_inff();
+  for (int p = 0; p < parts; ++p) m = fmaxf(m, w[p * step + 4096 + 2 * lane]);
+  float l = 0.0f;
+  float4 o[4] = {};
+#pragma unroll 2
+  for (int p = 0; p < parts; ++p) {
+    const float2 ml = *reinterpret_cast<const float2 *>(w + p * step + 4096 + 2 * lane);
+    const float a = __builtin_amdgcn_exp2f(ml.x - m);
+    l += a * ml.y;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float4 x = *reinterpret_cast<const float4 *>(w + p * step + ((4 * db + g) * 64 + lane) * 4);
+      o[g].x += a * x.x;
+      o[g].y += a * x.y;
+      o[g].z += a * x.z;
+      o[g].w += a * x.w;
+    }
+  }
+  const int q_row = qt * 32 * nwv + 32 * wave + (lane & 31);
+  if (q_row >= L) return;
+  const float inv = 1.0f / l;
+  const int b = bh / H, hh = bh - b * H;
+  uint16_t *orow = out + (static_cast<int64_t>(b) * L + q_row) * ldo + hh * kDh + 32 * db + 4 * (lane >> 5);
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+    *reinterpret_cast<uint2 *>(orow + 8 * g) =
+        make_uint2(pack_bf16x2(o[g].x * inv, o[g].y * inv), pack_bf16x2(o[g].z * inv, o[g].w * inv));
 }
 
 // vt[bh][d][l] = v[bh][l][d] for 64 tokens x 128 channels per workgroup, through LDS;
@@ -375,9 +451,55 @@ int attn_cu_count() {
   return v;
 }
 
+// How a call is cut up: the workgroup size, and a last round of few eight-wave items split over the keys.
+struct AttnPlan {
+  int nwv = 8;
+  AttnSplit split{0, 0, 0, nullptr};  // parts 0: not split
+  int64_t tail = 0;                   // split items
+};
+
+// Eight waves share each tile among more queries but run one workgroup per CU; of the four-wave workgroups two
+// run on a CU, or one, faster, when there are no more than CUs left. Relative time per key tile of a round of each
+// (us, fitted to B 1 and 4 at L = 768 to 4608 with 24 heads): 1.74, 1.9 and 1.3. Measured, four waves against
+// eight, us: B1 L 4608 274 / 251, B1 L 1536 45.7 / 42.4, B2 L 2300 145 / 135, B4 L 1536 127 / 142, B1 L 768 18 / 25.
+AttnPlan plan_attention(int64_t B, int64_t H, int64_t L, bool may_split) {
+  AttnPlan plan;
+  const int64_t cu = attn_cu_count(), n8 = B * H * cdiv(L, 256), n4 = B * H * cdiv(L, 128), rest = n4 % (2 * cu);
+  const double t8 = 1.74 * static_cast<double>(cdiv(n8, cu));
+  const double t4 = 1.9 * static_cast<double>(n4 / (2 * cu)) + (rest == 0 ? 0.0 : rest <= cu ? 1.3 : 1.9);
+  if (!(t8 < t4)) plan.nwv = 4;
+  // The eight-wave items of a last round of few run as ranges of keys on the idle CUs when that is estimated at least
+  // 4.8 % faster: the full rounds and a range's key tiles at 1.74 us each, 6 us for the second prologue and the merge,
+  // 0.085 us per range for its partial output. Measured, unsplit against split, 24 heads, us: B1 L 2816 (8 of 264
+  // items) 130.5 / 107.7, B2 L 1536 76.9 / 71.5, B1 L 5400 403 / 346, B1 L 4096 (half a round, two ranges) 207 / 196;
+  // estimated below the margin and not split: B4 L 1536 134 / 132, B3 L 1024 54 / 53, B2 L 1792 87.7 / 92.0.
+  const int64_t tail = n8 % cu, tiles = cdiv(L, kKT);
+  if (!may_split || n8 < cu || tail == 0) return plan;
+  const double now = (t8 < t4 ? t8 : t4) * static_cast<double>(tiles);
+  double best = 0.952 * now;
+  for (int64_t want = 2; want <= 16 && tail * want <= cu; ++want) {
+    const int64_t per = cdiv(tiles, want), parts = cdiv(tiles, per);
+    if (per < 2 || parts < 2) break;
+    const double us =
+        1.74 * static_cast<double>(n8 / cu * tiles + per) + 6.0 + 0.085 * static_cast<double>(tail * parts);
+    if (us < best) {
+      best = us;
+      plan.nwv = 8;
+      plan.tail = tail;
+      plan.split = {static_cast<int>(n8 - tail), static_cast<int>(parts), static_cast<int>(per), nullptr};
+    }
+  }
+  return plan;
+}
+
+int64_t split_bytes(const AttnPlan &plan) {
+  return plan.tail * plan.split.parts * plan.nwv * kPartialFloats * static_cast<int64_t>(sizeof(float));
+}
+
 template <bool VT>
 int attention_any(const char *what, const void *q, const void *k, const void *v, int64_t B, int64_t H, int64_t L,
-                  int64_t Dh, void *out, int64_t ldo, int dtype, void *stream) {
+                  int64_t Dh, void *out, int64_t ldo, int dtype, bool may_split, void *workspace,
+                  int64_t workspace_bytes, void *stream) {
   if (int e = check_heads(what, B, H, L, Dh, dtype)) return e;
   if (B == 0 || H == 0 || L == 0) return ok();
   if (!q || !k || !v || !out) return set_error(SELAS_EINVAL, "%s: null pointer", what);
@@ -385,38 +507,64 @@ int attention_any(const char *what, const void *q, const void *k, const void *v,
   if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 8) || ldo % 4)
     return set_error(SELAS_EUNSUPPORTED, "%s: q, k and the values must be 16-byte aligned, out rows 8-byte aligned", what);
   const float c2 = 1.4426950408889634f / sqrtf(static_cast<float>(Dh));  // log2(e) / sqrt(Dh)
-  auto launch = [&](auto kernel, int nwv) {
-    const int qtiles = static_cast<int>(cdiv(L, 32 * nwv));
-    const int64_t total = B * H * qtiles;
-    const int per_xcd = static_cast<int>(cdiv(total, 8));
-    kernel<<<dim3(static_cast<uint32_t>(per_xcd * 8)), dim3(64 * nwv), 0, static_cast<hipStream_t>(stream)>>>(
+  AttnPlan plan = plan_attention(B, H, L, may_split);
+  const int qtiles = static_cast<int>(cdiv(L, 32 * plan.nwv));
+  const int64_t total = B * H * qtiles;
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  auto launch = [&](auto kernel, int64_t whole, int64_t ranges) {
+    const int per_xcd = static_cast<int>(cdiv(whole, 8));
+    kernel<<<dim3(static_cast<uint32_t>(per_xcd * 8 + ranges)), dim3(64 * plan.nwv), 0, st>>>(
         static_cast<const uint16_t *>(q), static_cast<const uint16_t *>(k), static_cast<const uint16_t *>(v),
         static_cast<uint16_t *>(out), ldo, static_cast<int>(H), static_cast<int>(L), qtiles, per_xcd,
-        static_cast<int>(total), c2);
+        static_cast<int>(total), c2, plan.split);
   };
-  // Eight waves share each tile among more queries but run one workgroup per CU; of the four-wave workgroups two
-  // run on a CU, or one, faster, when there are no more than CUs left. Relative time per key tile of a round of each
-  // (us, fitted to B 1 and 4 at L = 768 to 4608 with 24 heads): 1.74, 1.9 and 1.3. Measured, four waves against
-  // eight, us: B1 L 4608 274 / 251, B1 L 1536 45.7 / 42.4, B2 L 2300 145 / 135, B4 L 1536 127 / 142, B1 L 768 18 / 25.
-  const int64_t cu = attn_cu_count(), n8 = B * H * cdiv(L, 256), n4 = B * H * cdiv(L, 128), rest = n4 % (2 * cu);
-  const double t8 = 1.74 * static_cast<double>(cdiv(n8, cu));
-  const double t4 = 1.9 * static_cast<double>(n4 / (2 * cu)) + (rest == 0 ? 0.0 : rest <= cu ? 1.3 : 1.9);
-  if (t8 < t4) launch(attn_fwd_kernel<8, VT>, 8);
-  else launch(attn_fwd_kernel<4, VT>, 4);
+  if constexpr (!VT) {
+    if (plan.split.parts) {
+      if (workspace_bytes < split_bytes(plan) || !workspace || !aligned(workspace, 16))
+        return set_error(SELAS_EINVAL, "%s: needs a 16-byte aligned workspace of %lld bytes", what,
+                         (long long)split_bytes(plan));
+      plan.split.partial = static_cast<float *>(workspace);
+      launch(attn_fwd_kernel<8, VT, true>, plan.split.whole, plan.tail * plan.split.parts);
+      if (int e = check_launch(what)) return e;
+      attn_merge_kernel<<<dim3(static_cast<uint32_t>(4 * plan.nwv * plan.tail)), dim3(64), 0, st>>>(
+          plan.split.partial, static_cast<uint16_t *>(out), ldo, static_cast<int>(H), static_cast<int>(L), qtiles,
+          plan.nwv, plan.split.whole, plan.split.parts);
+      return check_launch(what);
+    }
+  }
+  if (plan.nwv == 8) launch(attn_fwd_kernel<8, VT>, total, 0);
+  else launch(attn_fwd_kernel<4, VT>, total, 0);
   return check_launch(what);
 }
 }  // namespace
 
 extern "C" int selas_attention(const void *q, const void *k, const void *vt, int64_t B, int64_t H, int64_t L,
                                int64_t Dh, void *out, int64_t ldo, int dtype, void *stream) {
-  return attention_any<true>("attention", q, k, vt, B, H, L, Dh, out, ldo, dtype, stream);
+  return attention_any<true>("attention", q, k, vt, B, H, L, Dh, out, ldo, dtype, false, nullptr, 0, stream);
 }
 
 extern "C" int selas_attention_v(const void *q, const void *k, const void *v, int64_t B, int64_t H, int64_t L,
                                  int64_t Dh, void *out, int64_t ldo, int dtype, void *stream) {
   if (B >= 0 && H >= 0 && B * H > 65535)
     return set_error(SELAS_EUNSUPPORTED, "attention_v: more than 65535 heads");
-  return attention_any<false>("attention_v", q, k, v, B, H, L, Dh, out, ldo, dtype, stream);
+  return attention_any<false>("attention_v", q, k, v, B, H, L, Dh, out, ldo, dtype, false, nullptr, 0, stream);
+}
+
+extern "C" int selas_attention_workspace_bytes(int64_t B, int64_t H, int64_t L, int64_t *bytes) {
+  if (!bytes) return set_error(SELAS_EINVAL, "attention_workspace_bytes: null pointer");
+  *bytes = 0;
+  if (int e = check_heads("attention_workspace_bytes", B, H, L, kDh, SELAS_BF16)) return e;
+  if (B && H && L) *bytes = split_bytes(plan_attention(B, H, L, true));
+  return ok();
+}
+
+extern "C" int selas_attention_split(const void *q, const void *k, const void *v, int64_t B, int64_t H, int64_t L,
+                                     int64_t Dh, void *out, int64_t ldo, int dtype, void *workspace,
+                                     int64_t workspace_bytes, void *stream) {
+  if (B >= 0 && H >= 0 && B * H > 65535)
+    return set_error(SELAS_EUNSUPPORTED, "attention_split: more than 65535 heads");
+  return attention_any<false>("attention_split", q, k, v, B, H, L, Dh, out, ldo, dtype, true, workspace, workspace_bytes,
+                              stream);
 }
 
 extern "C" int selas_transpose_heads(const void *v, int64_t BH, int64_t L, int64_t Dh, void *vt, int dtype,
