@@ -84,8 +84,9 @@ int selas_nf4_encode(const float *w, int64_t n, int64_t blocksize, const float c
 /*
  * selas_nf4_encode of a tensor of dtype w_dtype (the exact conversion to fp32
  * is part of the kernel). 16-bit tensors need blocksize 64, 16-byte alignment
- * and a codebook in [-1, 1] whose midpoints ascend at least 1/16 apart
- * (otherwise SELAS_EUNSUPPORTED: convert to fp32 first).
+ * and a codebook whose midpoints ascend in (-1, 1), at most one in each of the 64
+ * buckets [b, b + 1) of 31.999 m + 32 and none but 0 within 2e-6 of an edge of its
+ * bucket (otherwise SELAS_EUNSUPPORTED: convert to fp32 first).
  */
 int selas_nf4_encode_typed(const void *w, int w_dtype, int64_t n, int64_t blocksize, const float code[16],
                            uint8_t *packed, float *absmax, void *stream);

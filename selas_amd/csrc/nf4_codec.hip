@@ -132,7 +132,8 @@ struct SearchTable {
 };
 __host__ __device__ __forceinline__ float bucket_of(float x) { return __builtin_fmaf(x, 31.999f, 32.0f); }
 // x = w * (1 / absmax) is within 2e-7 of w / absmax, and an entry within 16 ulp (1e-6) of its midpoint: closer than
-// this the elements are divided and searched exactly.
+// this the elements are divided and searched exactly. x meets only the entry of its own bucket, so search_table takes
+// no midpoint from which x could be off into the next bucket.
 constexpr float kNearMid = 2e-6f;
 
 // Blocks of 64, 16-byte aligned input. Eight lanes per block, eight consecutive elements per lane: 16-byte loads (fp32:
@@ -196,13 +197,18 @@ __global__ __launch_bounds__(kThreads) void nf4_encode_64(const void *__restrict
   }
 }
 
-// Fills `table` when nf4_encode_64 can use these midpoints: ascending, at most one per bucket.
+// Fills `table` when nf4_encode_64 can use these midpoints: ascending, at most one per bucket, and none within kNearMid
+// of its bucket's edges. (0 lies on an edge and may: x has the sign of w / absmax, and below 1e-6 bucket_of rounds to
+// the edge, whose bucket holds the entry.)
 bool search_table(const Mids15 &mids, SearchTable &table) {
   int bucket[15];
   for (int i = 0; i < 15; ++i) {
     if (!(mids.v[i] > -1.0f && mids.v[i] < 1.0f) || (i > 0 && !(mids.v[i] > mids.v[i - 1]))) return false;
     bucket[i] = static_cast<int>(bucket_of(mids.v[i]));
     if (i > 0 && bucket[i] == bucket[i - 1]) return false;
+    if (mids.v[i] != 0.0f && (static_cast<int>(bucket_of(mids.v[i] - kNearMid)) != bucket[i] ||
+                              static_cast<int>(bucket_of(mids.v[i] + kNearMid)) != bucket[i]))
+      return false;
   }
   int below = 0;
   for (int b = 0; b < 64; ++b) {

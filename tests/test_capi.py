@@ -7,6 +7,7 @@ import ctypes
 import re
 from pathlib import Path
 
+import numpy as np
 import pytest
 import torch
 
@@ -59,6 +60,48 @@ def test_invalid_arguments_are_reported_without_a_device_call():
     _lib.call("selas_nf4_dequant", null, null, 0, 64, _code(), null, _lib.BF16, null)
     _lib.call("selas_nf4_linear", null, 0, 64, 64, null, null, 64, _code(), 8, null, null, 8, _lib.BF16, null, 0,
               null)
+
+
+def nf4_bucket(x):
+    """bucket_of of the NF4 encoder (nf4_codec.hip) in fp32; the double product and sum are exact here."""
+    return np.float32(np.float64(np.float32(x)) * np.float64(np.float32(31.999)) + 32.0)
+
+
+def codebook_with_midpoint(mid):
+    """16 ascending codes in [-1, 1], at least 0.03 apart, one of whose fp32 midpoints is exactly ``mid``."""
+    mid = np.float32(mid)
+    c = np.linspace(-1, 1, 16, dtype=np.float32)
+    i = int(np.argmin(np.abs((c[1:] + c[:-1]) / 2 - mid)))
+    for step in range(1, 200):  # c[i] on a grid coarse enough for 2 mid - c[i] and the sum to be exact
+        c[i] = np.float32(np.round((float(mid) - 0.05) * 1024 + step % 20) / 1024)
+        c[i + 1] = np.float32(2 * np.float64(mid) - np.float64(c[i]))
+        if (c[i + 1] + c[i]) / np.float32(2) == mid and (np.diff(c) > 0.03).all():
+            return tuple(float(v) for v in c)
+    raise AssertionError(f"no codebook for midpoint {mid}")
+
+
+def edge_midpoints():
+    """(midpoints from which rounding reaches the next bucket of the encoder's table, midpoints safely inside)."""
+    bad, good = [], []
+    for b in (12, 20, 31, 33, 43, 50, 57):
+        x = np.float32((b - 32) / 31.999)
+        while nf4_bucket(x) >= b:
+            x = np.nextafter(x, np.float32(-2))
+        while nf4_bucket(x) < b:
+            x = np.nextafter(x, np.float32(2))
+        # x is the first float of bucket b
+        bad += [x, np.nextafter(x, np.float32(-2)), x + np.float32(1e-6), x - np.float32(1e-6)]
+        good += [x + np.float32(1e-5), x - np.float32(1e-5)]
+    return bad, good
+
+
+def test_nf4_encode_refuses_a_table_for_midpoints_at_a_bucket_edge():
+    # w * (1 / absmax) may round to the other side of the edge, where the table holds no entry of this midpoint.
+    x = ctypes.c_void_p(4096)
+    for mid in edge_midpoints()[0]:
+        with pytest.raises(_lib.Unsupported, match="midpoints"):
+            _lib.call("selas_nf4_encode_typed", x, _lib.BF16, 64, 64, _lib.code_array(codebook_with_midpoint(mid)), x, x,
+                      None)
 
 
 def test_python_wrappers_validate_like_the_reference():

@@ -11,9 +11,10 @@ import torch
 
 from oracle import int8_row as oi8
 from oracle import nf4 as onf4
-from selas_amd import codecs
+from selas_amd import _lib, codecs
 
 from .conftest import seeded
+from .test_capi import codebook_with_midpoint, edge_midpoints
 
 pytestmark = pytest.mark.gpu
 DTYPES = [torch.float32, torch.bfloat16, torch.float16]
@@ -121,3 +122,33 @@ def test_codebook_without_a_search_table():
     c = torch.tensor(code)
     idx = torch.bucketize(w.float() / a, (c[1:] + c[:-1]) / 2).view(-1, 2)
     assert torch.equal(e.parts["packed"].cpu(), ((idx[:, 0] << 4) | idx[:, 1]).to(torch.uint8))
+
+
+def takes_table(code):
+    w = torch.zeros(64, dtype=torch.bfloat16, device="cuda")
+    p, a = torch.zeros(32, dtype=torch.uint8, device="cuda"), torch.zeros(1, device="cuda")
+    try:
+        _lib.call("selas_nf4_encode_typed", w.data_ptr(), _lib.BF16, 64, 64, _lib.code_array(code), p.data_ptr(),
+                  a.data_ptr(), _lib.stream(w.device))
+    except _lib.Unsupported:
+        return False
+    return True
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_codebooks_with_midpoints_at_and_near_bucket_edges(dtype):
+    # The elements within 2 ulp of every midpoint of blocks of 400 magnitudes: byte-exact whether the codebook takes
+    # the table (midpoints 1e-5 inside an edge, a midpoint of 0, the spread codes) or not (midpoints at an edge).
+    bad, good = edge_midpoints()
+    a = (torch.rand(400, generator=seeded(9)) + 0.1).to(dtype).float().numpy()
+    spread = [tuple(float(c) for c in np.linspace(-0.97, 0.99, 16)), codebook_with_midpoint(0.0)]
+    for code, table in [(codebook_with_midpoint(m), False) for m in bad] + \
+            [(codebook_with_midpoint(m), True) for m in good] + [(c, True) for c in spread]:
+        assert takes_table(code) == table
+        v = near(a[:, None] * onf4.midpoints(code)[None, :], dtype, 2).view(5, 400, 15).permute(1, 0, 2).reshape(400, 75)
+        w = torch.cat([v[:, :63], torch.from_numpy(a)[:, None].to(dtype), v[:, 12:], torch.from_numpy(a)[:, None].to(dtype)],
+                      1)
+        e = codecs.encode_nf4("w", w.cuda(), code=code)
+        p, absmax = onf4.encode(w.float().numpy(), 64, code)
+        assert np.array_equal(e.parts["absmax"].cpu().numpy(), absmax)
+        assert (e.parts["packed"].cpu().numpy() == p).all(), code
