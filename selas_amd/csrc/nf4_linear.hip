@@ -355,6 +355,14 @@ struct GemvDesc {
   int64_t ldy;
 };
 
+// The power of two that brings a magnitude with these bf16 bits into [2^14, 2^15), exactly and with an exact inverse: k
+// stops at 126 (|x| below 2^-112, subnormal or 0 lands below 2^14), since 2^-127 is no normal number. 0 for Inf and NaN.
+__device__ __forceinline__ int x_scale_exp(uint32_t bits) {
+  const int e = static_cast<int>(bits >> 7);
+  return e == 0xff ? 0 : min(126, 14 + 127 - e);
+}
+__device__ __forceinline__ float pow2(int k) { return __uint_as_float(static_cast<uint32_t>(k + 127) << 23); }
+
 // A descriptor held in scalar registers (every field wave-uniform; n and ldy fit 32 bits).
 struct SDesc {
   const uint8_t *packed;
@@ -573,7 +581,7 @@ __global__ __launch_bounds__(64 * NW, 1) void nf4_gemv_stream(
   // or to zero), and the products with the fp16 codebook accumulate in fp32.
   // Each wave scales its fp32 partial sums back (exactly: a power of two) before
   // the waves' partials are added, so no row maximum over all of K is needed.
-  // Rows whose slice maximum is 0, Inf or NaN keep scale 1.
+  // Rows whose slice maximum is Inf or NaN keep scale 1.
   f16x8 xf[BPW][4];
   float inv[16];  // inverse scale of the row each partial-sum register holds
   {
@@ -591,10 +599,8 @@ __global__ __launch_bounds__(64 * NW, 1) void nf4_gemv_stream(
       }
     uint32_t mx = max(static_cast<uint32_t>(mx2.x), static_cast<uint32_t>(mx2.y));
     mx = max(mx, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mx), 32)));  // both halves of row c's slice
-    const unsigned e = (mx >> 7) & 0xffu;  // bf16 exponent field of the slice maximum
-    const int k = (e == 0u || e == 0xffu) ? 0 : 14 - (static_cast<int>(e) - 127);  // scale = 2^k
-    const float sc = __uint_as_float(static_cast<uint32_t>(max(-126, min(127, k)) + 127) << 23);
-    const float isc = __uint_as_float(static_cast<uint32_t>(max(-126, min(127, -k)) + 127) << 23);
+    const int k = x_scale_exp(mx);
+    const float sc = pow2(k), isc = pow2(-k);
 #pragma unroll
     for (int b = 0; b < BPW; ++b)
 #pragma unroll
@@ -820,7 +826,7 @@ __global__ __launch_bounds__(64 * NW, 1) void nf4_gemv_few(const uint16_t *__res
   float inv[MM];
 #pragma unroll
   for (int m = 0; m < MM; ++m) {
-    // |x| as bf16 magnitude bits; the scale 2^k brings the lane's largest into [2^14, 2^15) (1 for 0, Inf and NaN).
+    // |x| as bf16 magnitude bits; the scale 2^k brings the lane's largest into [2^14, 2^15) (x_scale_exp).
     uint32_t mx = 0;
 #pragma unroll
     for (int j = 0; j < KC; ++j)
@@ -830,10 +836,9 @@ __global__ __launch_bounds__(64 * NW, 1) void nf4_gemv_few(const uint16_t *__res
 #pragma unroll
         for (int i = 0; i < 4; ++i) mx = max(mx, max((w[i] >> 16) & 0x7fffu, w[i] & 0x7fffu));
       }
-    const unsigned e = mx >> 7;
-    const int k = (e == 0u || e == 0xffu) ? 0 : 14 - (static_cast<int>(e) - 127);
-    const float sc = __uint_as_float(static_cast<uint32_t>(max(-126, min(127, k)) + 127) << 23);
-    inv[m] = __uint_as_float(static_cast<uint32_t>(max(-126, min(127, -k)) + 127) << 23);
+    const int k = x_scale_exp(mx);
+    const float sc = pow2(k);
+    inv[m] = pow2(-k);
 #pragma unroll
     for (int j = 0; j < KC; ++j)
 #pragma unroll
