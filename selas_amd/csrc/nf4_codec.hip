@@ -3,6 +3,7 @@
 // Decode restates selas/codecs.py:178-199 (nf4_dequant_torch) and :207-228
 // (the Triton kernel): value = code[nibble] * absmax[block] in fp32, rounded
 // once to the output type. Encode restates selas/codecs.py:99-119.
+#include <algorithm>
 #include <cstring>
 
 #include "common.h"
@@ -90,9 +91,10 @@ int dequant_typed(const uint8_t *packed, const float *absmax, int64_t n_bytes, i
   if (bpb % 4 == 0 && aligned(packed, 4) && aligned(out, 16) && n_bytes >= 4 && n_bytes / 4 < (1ll << 31) - 4096) {
     const int64_t n4 = n_bytes / 4;
     const int64_t grid = cdiv(n4, kThreads * kDequantPer);
+    // The dwords past a first block of more than n4 do not exist: n4 gives the same quotients, 0, in 32 bits.
+    const FastDiv per_block = fast_div(static_cast<uint32_t>(std::min(bpb / 4, n4)));
     nf4_dequant_vec4<DT><<<dim3(static_cast<uint32_t>(grid)), dim3(kThreads), 0, stream>>>(
-        reinterpret_cast<const uint32_t *>(packed), absmax, static_cast<uint32_t>(n4),
-        fast_div(static_cast<uint32_t>(bpb / 4)), code, out);
+        reinterpret_cast<const uint32_t *>(packed), absmax, static_cast<uint32_t>(n4), per_block, code, out);
     done = n4 * 4;
   }
   if (done < n_bytes) {

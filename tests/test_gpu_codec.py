@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from oracle import nf4 as onf4
-from selas_amd import codecs
+from selas_amd import _lib, codecs
 
 from .conftest import seeded
 
@@ -118,3 +118,17 @@ def test_round_trip_at_full_linear_size(dev):
     assert (bits(out).reshape(-1) == onf4.decode(p_ref, a_ref, 64, out=onf4.BF16)).all()
     rel = (out.float().cpu() - w).norm() / w.norm()
     assert rel < 0.12
+
+
+@pytest.mark.parametrize("blocksize", [8192, 8200, 1 << 33, 1 << 35, (1 << 35) + 8, (1 << 62) + 64])
+def test_decode_of_a_part_of_one_block(dev, blocksize):
+    # A block of more elements than there are: one scale for all. Its dwords are counted in 64 bits (2^35 elements are
+    # 2^32 of them, and 2^35 + 8 one more).
+    packed = torch.randint(0, 256, (4096 + 3,), dtype=torch.uint8, generator=seeded(8))
+    n = min(packed.numel(), blocksize // 2)
+    absmax = torch.tensor([0.37])
+    p, a = packed.to(dev), absmax.to(dev)
+    out = torch.empty(2 * n, dtype=torch.bfloat16, device=dev)
+    _lib.call("selas_nf4_dequant", p.data_ptr(), a.data_ptr(), n, blocksize, _lib.code_array(codecs.NF4_CODE),
+              out.data_ptr(), _lib.BF16, _lib.stream(dev))
+    assert (bits(out) == oracle_bits(packed[:n], absmax, blocksize, torch.bfloat16)).all()
