@@ -390,7 +390,7 @@ int selas_attention(const void *q, const void *k, const void *vt, int64_t B, int
 /*
  * selas_attention with the values as v [B, H, L, Dh] in place of v^T: the
  * kernel transposes them on their way to the matrix cores. Same bits. At most
- * 65535 heads.
+ * 65535 heads. out may not overlap q, k or v.
  */
 int selas_attention_v(const void *q, const void *k, const void *v, int64_t B, int64_t H, int64_t L, int64_t Dh,
                       void *out, int64_t ldo, int dtype, void *stream);

@@ -26,6 +26,15 @@ def _heads(t: torch.Tensor, what: str) -> torch.Tensor:
     return t if t.is_contiguous() else t.contiguous()
 
 
+def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether the address ranges of two tensors (non-negative strides) meet."""
+    if a.numel() == 0 or b.numel() == 0:
+        return False
+    a0, b0 = a.data_ptr(), b.data_ptr()
+    ends = [t.element_size() * (1 + sum((n - 1) * s for n, s in zip(t.shape, t.stride()))) for t in (a, b)]
+    return a0 < b0 + ends[1] and b0 < a0 + ends[0]
+
+
 def transpose_heads(v: torch.Tensor) -> torch.Tensor:
     """v [B, H, L, Dh] -> [B, H, Dh, Lp] (contiguous), Lp = L rounded up to 64 tokens; the
     columns past L are zero."""
@@ -45,7 +54,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tens
     """softmax(q k^T / sqrt(Dh)) v over [B, H, L, Dh] -> [B, L, H * Dh].
 
     ``out``: optional [B, L, H * Dh] destination whose rows may be strided (e.g. the first
-    H * Dh columns of a wider buffer); it is returned."""
+    H * Dh columns of a wider buffer); it is returned. It may overlap v (v is then copied first), not q or k."""
     q, k = _heads(q, "attention"), _heads(k, "attention")
     if q.shape != k.shape or q.shape != v.shape or q.dtype != k.dtype or q.dtype != v.dtype:
         raise ValueError(f"attention: q {tuple(q.shape)} {q.dtype}, k {tuple(k.shape)} {k.dtype}, "
@@ -63,6 +72,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tens
         raise ValueError(f"attention: out must be [{b}, {l}, {h * d}] {q.dtype} on {q.device} with unit column "
                          f"stride and equally spaced rows, got {tuple(out.shape)} strides {out.stride()}")
     v = _heads(v, "attention")
+    if _overlap(out, v):  # workgroups store rows of out while others still read v
+        v = v.clone()
     size = ctypes.c_int64()
     with torch.cuda.device(dev):
         # 0 unless a last round of few workgroups is split over the keys; on the caller's stream, from torch's pool.

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 import torch
 
-from selas_amd import _lib, codecs, kernels
+from selas_amd import _lib, attention, codecs, kernels
 
 HEADER = Path(__file__).resolve().parent.parent / "include" / "selas_amd.h"
 
@@ -121,6 +121,13 @@ def test_python_wrappers_validate_like_the_reference():
     raw = codecs.encode_raw("b", torch.arange(6.0).view(2, 3), torch.float32)
     assert codecs.decode("raw", raw.parts, raw.meta, raw.shape, torch.float32).data_ptr() == raw.parts["data"].data_ptr()
     assert codecs.decoded_is_view("raw", "bfloat16", torch.bfloat16) and not codecs.decoded_is_view("nf4", None, torch.float32)
+
+
+def test_overlapping_address_ranges():
+    b = torch.zeros(100)
+    assert attention._overlap(b[:60], b[59:]) and not attention._overlap(b[:60], b[60:])
+    assert attention._overlap(b.view(10, 10)[:, 9:], b[95:]) and not attention._overlap(b.view(10, 10)[:9, :3], b[83:])
+    assert not attention._overlap(b[:0], b) and not attention._overlap(b, torch.zeros(100))
 
 
 def test_segment_stride_helpers():

@@ -42,3 +42,14 @@ def test_values_off_alignment_are_refused():
     odd = torch.empty(65 * 128 + 1, dtype=torch.bfloat16, device="cuda")[1:].view(1, 1, 65, 128)
     with pytest.raises(_lib.Unsupported):
         attention(q, k, odd.copy_(v))
+
+
+@pytest.mark.parametrize("l", [65, 768, 3000])
+def test_out_may_overlap_the_values(l):
+    q, k, v = (torch.randn(1, 1, l, 128, generator=seeded(l + i)).to(torch.bfloat16).cuda() for i in range(3))
+    want = attention(q, k, v)
+    buf = torch.zeros(l + 8, 128, dtype=torch.bfloat16, device="cuda")
+    for vo, oo in ((0, 0), (0, 8), (8, 0)):  # the same rows; 8 rows later, 8 earlier
+        buf[vo:vo + l] = v[0, 0]
+        got = attention(q, k, buf[vo:vo + l].view(1, 1, l, 128), out=buf[oo:oo + l].unsqueeze(0))
+        assert got.data_ptr() == buf[oo].data_ptr() and torch.equal(got, want)
