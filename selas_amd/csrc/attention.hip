@@ -264,7 +264,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
       m_run = raise ? mx : m_run;
     }
     // V^T fragments of the second product (db, kb, t2) = (i / 4, (i / 2) % 2, i % 2),
-    // the first kVAhead read before the exponentials, the rest kVAhead MFMAs ahead.
+    // each read kVAhead MFMAs ahead.
     constexpr int kVAhead = VT ? 8 : 6;  // two reads a fragment from V: 6 measured 1 % faster than 8, as 4
     bf16x8 vf[kVAhead];
 #pragma unroll
@@ -291,6 +291,16 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
       o[i / 4] = mfma32(vf[i % kVAhead], pb[(i / 2) % 2][i % 2], o[i / 4]);
       const int j = i + kVAhead;
       if (j < 16) vf[i % kVAhead] = vfrag(stage, j / 4, (j / 2) % 2, j % 2);
+    }
+    // The same order for the scheduler, which otherwise issues most of the transposing reads in fours right before
+    // their MFMAs: 240.7 -> 235.4 us for B1 L 4592.
+    if constexpr (!VT) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 2 * kVAhead, 0);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (i + kVAhead < 16) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      }
     }
     // The next tile has landed for this wave; the barrier then covers every wave
     // and orders this tile's LDS reads before the DMA that reuses its stage.
