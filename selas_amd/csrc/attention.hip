@@ -18,9 +18,9 @@
 //     register r then holds key 16*(r/8) + 8*h + r%8, i.e. 8 consecutive keys per
 //     MFMA k-step, as the V^T operand holds, transposed by the LDS reads
 //     (ds_read_b64_tr_b16). With v^T laid out by a kernel of its own (16-byte
-//     operand reads) the product itself ran 4 % faster at L = 4608, but that
-//     kernel cost 11 us there and half a call's time at L < 1024: 48.7 -> 42.1 us
-//     for B1 L 1536, 258.5 -> 254.6 us for B1 L 4608.
+//     operand reads) the product itself ran 1 % faster at L = 4592, 241 us, but
+//     that kernel takes 10 us there and half a call's time at L < 1024. Call
+//     against call: 258.6 -> 247.5 us for B1 L 4592, 53.6 -> 40.2 for B1 L 1536.
 // LDS tiles are XOR-swizzled in 16-byte chunks so that the fragment reads (16
 // lanes per LDS cycle) hit 16 distinct 4-bank groups.
 // Any sequence length: key and query rows past L read as zeros (buffer range),
@@ -91,7 +91,10 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
                                                                AttnSplit sp) {
   constexpr int kQT = 32 * NWV;  // queries per workgroup
   constexpr int KJ = 16 / NWV;   // DMA instructions per wave and tile, for K and for V^T each
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * kStageBytes];
+  // An array per stage: the compiler then knows that reads of one stage do not touch the DMA into the other. With one
+  // array for both it waited for the next tile's loads before the first transposing read of a tile: 254 -> 250 us for
+  // B1 L 4592 on inputs that come from HBM.
+  __shared__ __attribute__((aligned(1024))) uint8_t smem0[kStageBytes], smem1[kStageBytes];
   // Work item t = (b % 8) * per_xcd + b / 8: each XCD takes a contiguous range,
   // so the query tiles of one head share that head's K and V^T in its L2.
   // Split: the whole items first, then the ranges, a range's parts on different XCDs.
@@ -148,7 +151,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
     }
   }
   auto issue = [&](int stage, int kt) {
-    uint8_t *base = smem + stage * kStageBytes;
+    uint8_t *base = stage ? smem1 : smem0;
     const uint32_t key0 = static_cast<uint32_t>(kt) * kKT;
 #pragma unroll
     for (int j = 0; j < KJ; ++j) load_lds16(kr, base + (KJ * wave + j) * 1024, k_voff[j], key0 * 256u);
@@ -161,7 +164,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
   auto kfrag = [&](int stage, int kb, int s) {
     const int r = 32 * kb + krow;
     const int cc = 2 * s + h;
-    return *reinterpret_cast<const bf16x8 *>(smem + stage * kStageBytes + r * 256 + ((cc ^ (r & 15)) << 4));
+    return *reinterpret_cast<const bf16x8 *>((stage ? smem1 : smem0) + r * 256 + ((cc ^ (r & 15)) << 4));
   };
   // V as the A operand of O^T += V^T P^T: lane (c, h) needs channel 32db + c of the keys 32kb + 16t + 8h .. +8.
   // ds_read_b64_tr_b16 transposes on the way: the 16 lanes of a group each address 4 channels of one of 4 keys (lane
@@ -174,7 +177,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
     for (int db = 0; db < 4; ++db) v_rd[db] = (8 * h + r) * 256 + ((db ^ r) << 6) + x * 16 + 8 * (lane & 1);
   }
   auto vfrag = [&](int stage, int db, int kb, int t2) {
-    uint8_t *vs = smem + stage * kStageBytes + kTileBytes;
+    uint8_t *vs = (stage ? smem1 : smem0) + kTileBytes;
     if constexpr (VT) {
       const int d = 32 * db + c;
       const int cc = 4 * kb + 2 * t2 + h;
