@@ -396,13 +396,14 @@ int selas_attention_v(const void *q, const void *k, const void *v, int64_t B, in
                       void *out, int64_t ldo, int dtype, void *stream);
 
 /*
- * selas_attention_v where a last round of few 256-query items leaves most CUs
- * idle: those items run as ranges of keys on the idle CUs, their fp32 partial
- * outputs are kept in `workspace` (device memory, 16-byte aligned, at least
- * selas_attention_workspace_bytes) and added in key order. The choice and the
- * size depend on B, H, L and the CU count only; with a size of 0 the call is
- * selas_attention_v, bit for bit. A workspace that is missing or too small is
- * SELAS_EINVAL, with nothing launched.
+ * selas_attention_v where the 256-query items of an image leave a last round of
+ * few, and most CUs idle: those items run as ranges of keys on the idle CUs, their
+ * fp32 partial outputs are kept in `workspace` (device memory, 16-byte aligned, at
+ * least selas_attention_workspace_bytes) and added in key order. The choice depends
+ * on H, L and the CU count only, so an image has the same bits in every batch; the
+ * size is B times an image's. With a size of 0 the call is selas_attention_v, bit
+ * for bit. A workspace that is missing or too small is SELAS_EINVAL, with nothing
+ * launched.
  */
 int selas_attention_split(const void *q, const void *k, const void *v, int64_t B, int64_t H, int64_t L, int64_t Dh,
                           void *out, int64_t ldo, int dtype, void *workspace, int64_t workspace_bytes, void *stream);

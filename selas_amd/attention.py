@@ -4,8 +4,9 @@ The reference calls ``F.scaled_dot_product_attention(q, k, v)`` on q, k, v
 [B, H, L, Dh] and returns ``out.transpose(1, 2).reshape(B, L, H * Dh)``.
 ``attention`` computes the same with one fused kernel that writes the
 [B, L, H * Dh] layout directly (the transpose copy disappears) and reads v as it
-is. Where the last round of workgroups is a small one it is split over the keys,
-by B, H, L and the CU count only. ``transpose_heads`` lays v out as the C entry
+is. Where an image's last round of workgroups is a small one it is split over the
+keys, by H, L and the CU count only: an image has the same bits in every batch.
+``transpose_heads`` lays v out as the C entry
 ``selas_attention`` takes it. Any sequence length runs; shapes outside the kernel (head
 dim other than 128, dtypes other than bf16) raise ``Unsupported``;
 ``flux.attention`` then runs SDPA, as the reference.

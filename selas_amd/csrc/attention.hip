@@ -33,6 +33,7 @@
 // ran 25 % slower, because a lone wave cannot overlap its softmax with MFMAs.
 // Eight waves per workgroup (one workgroup per CU) share each tile's DMA among
 // 256 queries instead of 128, which cuts the LDS traffic per query by a tenth.
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -71,11 +72,15 @@ __device__ __forceinline__ uint32_t pack_probs(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
-// Items from `whole` on run as `parts` ranges of `per` key tiles each (selas_attention_split); a range leaves each
-// wave's output, not yet divided, and its queries' maxima and sums in `partial`.
+// Of every image's `items` work items the last `tail` run as `parts` ranges of `per` key tiles each
+// (selas_attention_split); a range leaves each wave's output, not yet divided, and its queries' maxima and sums in
+// `partial`.
 struct AttnSplit {
-  int whole, parts, per;
+  int items, tail, parts, per;
   float *partial;
+  // Work item of whole item w, of split item s.
+  __host__ __device__ int whole_item(int w) const { return w + w / (items - tail) * tail; }
+  __host__ __device__ int split_item(int s) const { return (s / tail + 1) * items - tail + s % tail; }
 };
 // Per wave and range: 64 x 64 outputs in the order of the registers (1 KiB per store instruction), then per lane the
 // running maximum and the sum.
@@ -102,12 +107,14 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
   if constexpr (SPLIT) {
     if (static_cast<int>(blockIdx.x) >= 8 * per_xcd) {
       range = blockIdx.x - 8 * per_xcd;
-      t = sp.whole + range / sp.parts;
-    } else if (t >= sp.whole) {
-      return;
+      t = sp.split_item(range / sp.parts);
+    } else {
+      if (t >= total) return;
+      t = sp.whole_item(t);
     }
+  } else {
+    if (t >= total) return;
   }
-  if (t >= total) return;
   const int bh = t / qtiles, qt = t - bh * qtiles;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -349,13 +356,13 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *_
 
 // The split items' outputs from their ranges, added in key order: a workgroup of one wave per 32 queries and 32
 // channels, in the lane order of attn_fwd_kernel. Bounded by the reads of the partial outputs (L2, Infinity Cache).
-__global__ __launch_bounds__(64) void attn_merge_kernel(const float *__restrict__ partial, uint16_t *__restrict__ out,
-                                                        int64_t ldo, int H, int L, int qtiles, int nwv, int whole,
-                                                        int parts) {
+__global__ __launch_bounds__(64) void attn_merge_kernel(uint16_t *__restrict__ out,
+                                                        int64_t ldo, int H, int L, int qtiles, int nwv,
+                                                        AttnSplit sp) {
   const int lane = threadIdx.x, db = blockIdx.x & 3, wave = (blockIdx.x >> 2) % nwv, item = (blockIdx.x >> 2) / nwv;
-  const int t = whole + item, bh = t / qtiles, qt = t - bh * qtiles;
+  const int t = sp.split_item(item), bh = t / qtiles, qt = t - bh * qtiles, parts = sp.parts;
   const int64_t step = static_cast<int64_t>(nwv) * kPartialFloats;  // from one range to the next
-  const float *w = partial + (static_cast<int64_t>(item) * parts * nwv + wave) * kPartialFloats;
+  const float *__restrict__ w = sp.partial + (static_cast<int64_t>(item) * parts * nwv + wave) * kPartialFloats;
   float m = -__builtin_inff();
   for (int p = 0; p < parts; ++p) m = fmaxf(m, w[p * step + 4096 + 2 * lane]);
   float l = 0.0f;
@@ -464,46 +471,53 @@ int attn_cu_count() {
 // How a call is cut up: the workgroup size, and a last round of few eight-wave items split over the keys.
 struct AttnPlan {
   int nwv = 8;
-  AttnSplit split{0, 0, 0, nullptr};  // parts 0: not split
-  int64_t tail = 0;                   // split items
+  AttnSplit split{0, 0, 0, 0, nullptr};  // parts 0: not split
 };
 
 // Eight waves share each tile among more queries but run one workgroup per CU; of the four-wave workgroups two
 // run on a CU, or one, faster, when there are no more than CUs left. Relative time per key tile of a round of each
-// (us, fitted to B 1 and 4 at L = 768 to 4608 with 24 heads): 1.74, 1.9 and 1.3. Measured, four waves against
-// eight, us: B1 L 4608 274 / 251, B1 L 1536 45.7 / 42.4, B2 L 2300 145 / 135, B4 L 1536 127 / 142, B1 L 768 18 / 25.
+// (us, fitted to B 1 and 4 at L = 768 to 4608 with 24 heads): 1.74, 1.9 and 1.3. Measured when fitted, four waves
+// against eight, us: B1 L 4608 274 / 251, B1 L 1536 45.7 / 42.4, B2 L 2300 145 / 135, B4 L 1536 127 / 142, B1 L 768
+// 18 / 25.
+constexpr double kTile8 = 1.74, kTile4 = 1.9, kTile4Half = 1.3;
+
+double rounds8(int64_t B, int64_t H, int64_t L) {
+  return kTile8 * static_cast<double>(cdiv(B * H * cdiv(L, 256), static_cast<int64_t>(attn_cu_count())));
+}
+double rounds4(int64_t B, int64_t H, int64_t L) {
+  const int64_t cu = attn_cu_count(), n4 = B * H * cdiv(L, 128), rest = n4 % (2 * cu);
+  return kTile4 * static_cast<double>(n4 / (2 * cu)) + (rest == 0 ? 0.0 : rest <= cu ? kTile4Half : kTile4);
+}
+
+// The eight-wave items that an image has beyond full rounds of the CUs run as ranges of keys on the idle CUs. Whether
+// and how is decided for one image, from H, L and the CU count: an image has the same bits in every batch. So the cut
+// has to serve two to four images too, whose items fill rounds that one image leaves partly idle: at most an eighth of
+// a round is cut up per full round, into at most half a round of ranges. Not where four-wave workgroups need less (L
+// 2688: 92 us), and not for fewer than 40 key tiles (a range's prologue, its partial output and the merge take 8 us).
+// Unsplit / split, us, batch 1 to 4, 24 heads: L 2700 125 / 104, 206 / 188, 308 / 271, 392 / 359; L 3072 138 / 119,
+// 232 / 221, 343 / 334, 446 / 438 (six images 639 / 651, eight 829 / 873); L 5632 406 / 353, 764 / 682; L 6144
+// 448 / 425, 834 / 802. Past the line: L 3328 (56 items over one round) in 3 ranges 151 / 137, 257 / 270, in 2
+// 151 / 144, 257 / 254, 382 / 395; L 4096 (128) 196 / 194, 361 / 379; 32 heads, L 2100 (33 key tiles) 97 / 88 and, batch
+// 4, 304 / 312.
+AttnSplit plan_split(int64_t H, int64_t L) {
+  AttnSplit split{0, 0, 0, 0, nullptr};
+  const int64_t cu = attn_cu_count(), items = H * cdiv(L, 256), tail = items % cu, full = items / cu, tiles = cdiv(L, kKT);
+  if (tail == 0 || 8 * tail > cu * full || 4 * tail > cu || tiles < 40) return split;
+  const int64_t per = cdiv(tiles, std::min<int64_t>(8, cu / (2 * tail))), parts = cdiv(tiles, per);
+  const double cut = kTile8 * (static_cast<double>(full) + 1.0 / static_cast<double>(parts));
+  if (cut > 0.95 * std::min(rounds8(1, H, L), rounds4(1, H, L))) return split;
+  return {static_cast<int>(items), static_cast<int>(tail), static_cast<int>(parts), static_cast<int>(per), nullptr};
+}
+
 AttnPlan plan_attention(int64_t B, int64_t H, int64_t L, bool may_split) {
   AttnPlan plan;
-  const int64_t cu = attn_cu_count(), n8 = B * H * cdiv(L, 256), n4 = B * H * cdiv(L, 128), rest = n4 % (2 * cu);
-  const double t8 = 1.74 * static_cast<double>(cdiv(n8, cu));
-  const double t4 = 1.9 * static_cast<double>(n4 / (2 * cu)) + (rest == 0 ? 0.0 : rest <= cu ? 1.3 : 1.9);
-  if (!(t8 < t4)) plan.nwv = 4;
-  // The eight-wave items of a last round of few run as ranges of keys on the idle CUs when that is estimated at least
-  // 4.8 % faster: the full rounds and a range's key tiles at 1.74 us each, 6 us for the second prologue and the merge,
-  // 0.085 us per range for its partial output. Measured, unsplit against split, 24 heads, us: B1 L 2816 (8 of 264
-  // items) 130.5 / 107.7, B2 L 1536 76.9 / 71.5, B1 L 5400 403 / 346, B1 L 4096 (half a round, two ranges) 207 / 196;
-  // estimated below the margin and not split: B4 L 1536 134 / 132, B3 L 1024 54 / 53, B2 L 1792 87.7 / 92.0.
-  const int64_t tail = n8 % cu, tiles = cdiv(L, kKT);
-  if (!may_split || n8 < cu || tail == 0) return plan;
-  const double now = (t8 < t4 ? t8 : t4) * static_cast<double>(tiles);
-  double best = 0.952 * now;
-  for (int64_t want = 2; want <= 16 && tail * want <= cu; ++want) {
-    const int64_t per = cdiv(tiles, want), parts = cdiv(tiles, per);
-    if (per < 2 || parts < 2) break;
-    const double us =
-        1.74 * static_cast<double>(n8 / cu * tiles + per) + 6.0 + 0.085 * static_cast<double>(tail * parts);
-    if (us < best) {
-      best = us;
-      plan.nwv = 8;
-      plan.tail = tail;
-      plan.split = {static_cast<int>(n8 - tail), static_cast<int>(parts), static_cast<int>(per), nullptr};
-    }
-  }
+  if (may_split) plan.split = plan_split(H, L);
+  if (plan.split.parts == 0 && rounds8(B, H, L) >= rounds4(B, H, L)) plan.nwv = 4;
   return plan;
 }
 
-int64_t split_bytes(const AttnPlan &plan) {
-  return plan.tail * plan.split.parts * plan.nwv * kPartialFloats * static_cast<int64_t>(sizeof(float));
+int64_t split_bytes(const AttnPlan &plan, int64_t B) {
+  return B * plan.split.tail * plan.split.parts * plan.nwv * kPartialFloats * static_cast<int64_t>(sizeof(float));
 }
 
 template <bool VT>
@@ -526,19 +540,18 @@ int attention_any(const char *what, const void *q, const void *k, const void *v,
     kernel<<<dim3(static_cast<uint32_t>(per_xcd * 8 + ranges)), dim3(64 * plan.nwv), 0, st>>>(
         static_cast<const uint16_t *>(q), static_cast<const uint16_t *>(k), static_cast<const uint16_t *>(v),
         static_cast<uint16_t *>(out), ldo, static_cast<int>(H), static_cast<int>(L), qtiles, per_xcd,
-        static_cast<int>(total), c2, plan.split);
+        static_cast<int>(whole), c2, plan.split);
   };
   if constexpr (!VT) {
     if (plan.split.parts) {
-      if (workspace_bytes < split_bytes(plan) || !workspace || !aligned(workspace, 16))
-        return set_error(SELAS_EINVAL, "%s: needs a 16-byte aligned workspace of %lld bytes", what,
-                         (long long)split_bytes(plan));
+      const int64_t bytes = split_bytes(plan, B), tail = B * plan.split.tail;
+      if (workspace_bytes < bytes || !workspace || !aligned(workspace, 16))
+        return set_error(SELAS_EINVAL, "%s: needs a 16-byte aligned workspace of %lld bytes", what, (long long)bytes);
       plan.split.partial = static_cast<float *>(workspace);
-      launch(attn_fwd_kernel<8, VT, true>, plan.split.whole, plan.tail * plan.split.parts);
+      launch(attn_fwd_kernel<8, VT, true>, total - tail, tail * plan.split.parts);
       if (int e = check_launch(what)) return e;
-      attn_merge_kernel<<<dim3(static_cast<uint32_t>(4 * plan.nwv * plan.tail)), dim3(64), 0, st>>>(
-          plan.split.partial, static_cast<uint16_t *>(out), ldo, static_cast<int>(H), static_cast<int>(L), qtiles,
-          plan.nwv, plan.split.whole, plan.split.parts);
+      attn_merge_kernel<<<dim3(static_cast<uint32_t>(4 * plan.nwv * tail)), dim3(64), 0, st>>>(
+          static_cast<uint16_t *>(out), ldo, static_cast<int>(H), static_cast<int>(L), qtiles, plan.nwv, plan.split);
       return check_launch(what);
     }
   }
@@ -564,7 +577,7 @@ extern "C" int selas_attention_workspace_bytes(int64_t B, int64_t H, int64_t L, 
   if (!bytes) return set_error(SELAS_EINVAL, "attention_workspace_bytes: null pointer");
   *bytes = 0;
   if (int e = check_heads("attention_workspace_bytes", B, H, L, kDh, SELAS_BF16)) return e;
-  if (B && H && L) *bytes = split_bytes(plan_attention(B, H, L, true));
+  if (B && H && L) *bytes = split_bytes(plan_attention(B, H, L, true), B);
   return ok();
 }
 

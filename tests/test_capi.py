@@ -191,6 +191,23 @@ def test_split_workspace_is_sized_from_shapes_only():
         _ws_query([(64, 64, 64)] * 5)
 
 
+def test_attention_is_split_image_by_image():
+    # Whether an image's last items are cut over the keys depends on H, L and the CU count, so a batch needs the
+    # workspace of its images: 24 heads x 2816 tokens are 264 items for 256 CUs, 8 of them in 8 ranges of 8 waves.
+    def query(b, h, l):
+        out = ctypes.c_int64(-1)
+        _lib.call("selas_attention_workspace_bytes", b, h, l, ctypes.byref(out))
+        return out.value
+
+    wave = (64 * 64 + 2 * 64) * 4
+    assert query(1, 24, 2816) == 8 * 8 * 8 * wave and query(1, 24, 3072) == 32 * 4 * 8 * wave
+    for l in (1, 768, 1536, 2304, 2560, 2688, 3328, 4096, 4592, 4608):
+        assert query(1, 24, l) == query(2, 24, l) == query(4, 24, l) == 0, l
+    for h in (1, 2, 24, 25, 48, 100, 257, 1000, 1281):
+        for l in range(16, 20000, 61):
+            assert query(3, h, l) == 3 * query(1, h, l) and query(8, h, l) == 8 * query(1, h, l), (h, l)
+
+
 def test_split_launch_without_its_workspace_is_refused_before_any_device_call():
     # A split shape with no (or too small, or misaligned) workspace is an argument error, never an unsplit launch.
     x = ctypes.c_void_p(1 << 20)

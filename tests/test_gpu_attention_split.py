@@ -69,6 +69,18 @@ def test_against_64_bits_and_the_unsplit_call(b, h, l):
     assert d.norm() <= 4e-3 * u.double()[:, -min(l, 512):, -128:].norm()
 
 
+# Lengths that are cut (2816, 3000, 5400 tokens), and one that fills no round alone but one and an eighth in pairs.
+@pytest.mark.parametrize("b,h,l", [(2, 24, 1536), (3, 24, 2816), (4, 24, 3000), (2, 24, 5400), (3, 32, 2561), (2, 1, 65556)])
+def test_an_image_has_the_same_bits_in_every_batch(b, h, l):
+    q, k, v = inputs(b, h, l, 11)
+    y = attention(q, k, v)
+    for i in range(b):
+        assert torch.equal(y[i:i + 1], attention(q[i:i + 1], k[i:i + 1], v[i:i + 1])), i
+    if l < 4096:
+        check(y, q, k, v, b - 1, h - 1)
+        check(y, q, k, v, 0, h - 1)
+
+
 def test_a_range_without_weight():
     q, k, v = inputs(1, 24, 2816, 3)
     q[..., 0] = 1.0
