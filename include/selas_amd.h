@@ -130,9 +130,11 @@ int selas_int8_row_encode_typed(const void *w, int w_dtype, int64_t rows, int64_
  * load; its operand is the reference's decoded weight bf16(code*absmax) bit for
  * bit. M <= 32 runs a skinny dequant-GEMM that multiplies x by the codes and
  * scales the fp32 block sums by absmax (for K = 1024, 2048, 3072 in fp16 after
- * an exact power-of-two rescale of each row of x; otherwise in bf16 with codes
- * split into two bf16 terms); it agrees with the decoded-weight product to the
- * rounding of the decoded weight. Every output of the tiled GEMM sums K in
+ * an exact power-of-two rescale of parts of each row of x, by one kernel for M <= 2
+ * and another up to 32; otherwise in bf16 with codes split into two bf16 terms); it
+ * agrees with the decoded-weight product to the rounding of the decoded weight. A
+ * row's bits do not depend on the other rows; they may differ in the last bit
+ * between M <= 2, M <= 32 and the tiled GEMM. Every output of the tiled GEMM sums K in
  * one order, whatever M and the tile height, except where a launch splits its
  * last round of tiles over K (long K and a last round of few tiles, e.g.
  * M 6144, N 3072, K 15360): those tiles' K ranges are summed in fp32 by a

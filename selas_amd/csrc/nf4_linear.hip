@@ -6,13 +6,15 @@
 //
 // Kernels, chosen from M and K:
 //   * M <= 32 (hoisted adaLN modulation linears, M = number of steps), HBM-bound:
-//     nf4_gemv_few (M <= 2) and nf4_gemv_stream for K = 1024, 2048, 3072 (one launch can cover many
-//     weights), nf4_gemv_kernel for other K. Both multiply x by the codes on
-//     MFMA and apply the block's fp32 absmax to the fp32 block partial sums;
-//     codes come from bank-replicated LDS tables indexed by the packed byte.
+//     nf4_gemv_few (M <= 2, v_dot2) and nf4_gemv_stream (MFMA) for K = 1024, 2048,
+//     3072 (one launch can cover many weights), nf4_gemv_kernel (MFMA) for other K.
+//     They multiply x by the codes and apply the block's fp32 absmax to the fp32
+//     block partial sums; codes come from bank-replicated LDS tables indexed by the
+//     packed byte.
 //   * M > 32 (block linears, M = tokens), MFMA-bound: nf4_gemm_kernel.
-//     256x256 output tile per workgroup, 4 waves, each wave owns 64 output
-//     columns for all 256 rows. x tiles are staged through LDS (XOR-swizzled
+//     Output tiles of 256, 224 or 192 rows x 256 columns, or of 256, 192 or 128
+//     rows x 128 columns where those leave CUs idle (plan_gemm); 4 waves, each
+//     owning a quarter of the columns for all rows. x tiles are staged through LDS (XOR-swizzled
 //     16-byte chunks, three stages in flight); weight codes go straight from
 //     HBM to registers and are decoded to the bit-exact reference operand
 //     bf16(code[nibble] * absmax) with a per-block 16-entry product table and
@@ -1328,12 +1330,10 @@ __device__ __forceinline__ void interleave_substep() {
 // Fused-dequant GEMM. A workgroup is NW waves side by side along N; a wave
 // owns MB*32 rows x CB*32 columns of the output (MB*CB tiles of 32x32, 16
 // accumulator registers each):
-//   MB=8, CB=2, NW=4: 256 x 256 tile, 256 accumulators, one wave per SIMD;
-//                     each decoded weight fragment serves 8 MFMAs.
-//   MB=4, CB=2, NW=8: 128 x 512 tile, 128 accumulators, two waves per SIMD
-//                     (one wave's waits overlap the other's MFMAs); each
-//                     decoded fragment serves 4 MFMAs.
-// Either way the workgroup reads 128 KiB of x fragments from LDS per K block.
+//   CB=2, MB=8, 7, 6: 256, 224 or 192 rows x 256 columns, up to 256 accumulators,
+//                     one wave per SIMD; a decoded weight fragment serves MB MFMAs.
+//   CB=1, MB=8, 6, 4: 256, 192 or 128 rows x 128 columns where the wide tiles leave
+//                     CUs idle; half the MFMAs per x fragment read from LDS.
 //
 // Grid: workgroup b runs on XCD b % 8; tile t = (b % 8) * per_xcd + b / 8
 // gives each XCD a contiguous range of tiles. Within a problem the tiles go in

@@ -51,6 +51,20 @@ def test_alone_and_in_a_group(m, k):
     check(nf4_linear(x, *no_bias), x, ws[3][1], 0.0)
 
 
+@pytest.mark.parametrize("k", [1024, 3072])
+def test_a_row_has_the_same_bits_on_either_side_of_the_third(k):
+    # Rows do not see each other: M = 1 gives a row the bits of M = 2, and M = 3 those of M = 32. Between the two kernels
+    # only the order of the fp32 sums and the granularity of x's scale differ, about 1e-6 of a sum: an output differs
+    # where that crosses a bf16 rounding, by 2^-8 of itself, so with 1 % of such outputs by 4e-4 in the 2-norm.
+    w, _, _ = weight(1500, k, 21)
+    x = torch.randn(32, k, generator=seeded(k)).to(torch.bfloat16).cuda()
+    one, two, three, all32 = (nf4_linear(x[:m], *w) for m in (1, 2, 3, 32))
+    assert torch.equal(one, two[:1]) and torch.equal(nf4_linear(x[1:2], *w), two[1:])
+    assert torch.equal(three, all32[:3]) and torch.equal(nf4_linear(x[29:], *w), all32[29:])
+    d = (two.double() - three[:2].double()).norm()
+    assert d <= 4e-4 * three[:2].double().norm()
+
+
 def test_one_round_and_a_part():
     w, ref, b = weight(18432, 3072, 3)
     x = torch.nn.functional.silu(torch.randn(1, 3072, generator=seeded(5))).to(torch.bfloat16).cuda()
