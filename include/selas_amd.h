@@ -54,7 +54,7 @@ extern "C" {
 /* Message of the last failed call on this thread ("" if none). */
 const char *selas_last_error(void);
 
-/* ABI version of this header (bumped on any signature change). */
+/* ABI version of this header (bumped on any new or changed signature). */
 int selas_abi_version(void);
 
 /* ------------------------------------------------------------------ codec */

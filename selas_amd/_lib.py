@@ -14,7 +14,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "libselas_amd.so"
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 OK, EINVAL, EUNSUPPORTED, EHIP = 0, 1, 2, 3
 F32, F16, BF16 = 0, 1, 2
@@ -107,7 +107,9 @@ def load() -> ctypes.CDLL:
             if lib.selas_abi_version() != ABI_VERSION:
                 raise RuntimeError(f"{LIB_PATH} has ABI {lib.selas_abi_version()}, expected {ABI_VERSION}: rebuild it")
             for name, args in SIGNATURES.items():
-                fn = getattr(lib, name)
+                fn = getattr(lib, name, None)
+                if fn is None:
+                    raise RuntimeError(f"{LIB_PATH} has no {name}: rebuild it")
                 fn.restype = ctypes.c_int
                 fn.argtypes = args
             _lib = lib

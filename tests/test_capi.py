@@ -31,6 +31,16 @@ def test_library_exports_every_declared_symbol():
     assert lib.selas_abi_version() == _lib.ABI_VERSION
 
 
+def test_a_library_of_another_version_is_to_be_rebuilt(monkeypatch):
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "SIGNATURES", {**_lib.SIGNATURES, "selas_from_a_later_version": []})
+    with pytest.raises(RuntimeError, match="selas_from_a_later_version: rebuild it"):
+        _lib.load()
+    monkeypatch.setattr(_lib, "ABI_VERSION", _lib.ABI_VERSION + 1)
+    with pytest.raises(RuntimeError, match="expected .*: rebuild it"):
+        _lib.load()
+
+
 def _code():
     return _lib.code_array(codecs.NF4_CODE)
 
