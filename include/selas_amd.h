@@ -215,6 +215,15 @@ int selas_linear_workspace_bytes(const selas_nf4_gemm_problem *problems, int64_t
                                  int64_t *bytes);
 
 /*
+ * Rows and columns of the output tiles that the same launch runs in (0 and 0 where a
+ * skinny kernel takes it); the arguments as for selas_linear_workspace_bytes. It says
+ * which kernel a size runs, for measurements and tests; the bits do not depend on it.
+ * No counterpart in the reference.
+ */
+int selas_linear_tile(const selas_nf4_gemm_problem *problems, int64_t count, int codec, int64_t *rows,
+                      int64_t *cols);
+
+/*
  * Quantized linear forward y = x W^T + bias with W an int8_row [N, K] weight
  * (q int8 [N, K] row-major, 16-byte aligned; scale fp32 [N]); x, bias, y and
  * dtype as for selas_nf4_linear.

@@ -33,6 +33,7 @@ SIGNATURES: dict[str, list] = {
     "selas_nf4_linear_grouped": [_P, _I64, _I64, _I64, _P, _I64, _I64, _I64, _F16x, _INT, _P],
     "selas_nf4_linear_batched": [_P, _I64, _I64, _F16x, _INT, _P, _I64, _P],
     "selas_linear_workspace_bytes": [_P, _I64, _INT, ctypes.POINTER(ctypes.c_int64)],
+    "selas_linear_tile": [_P, _I64, _INT, ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64)],
     "selas_nf4_linear_grouped_static": [_P, _I64, _I64, _I64, _P, _I64, _I64, _F16x, _INT, _P],
     "selas_int8_row_dequant": [_P, _P, _I64, _I64, _P, _INT, _P],
     "selas_int8_row_encode": [_P, _I64, _I64, _P, _P, _P],

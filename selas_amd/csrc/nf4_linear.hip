@@ -2100,6 +2100,10 @@ GemmPlan plan_wide_tiles(const GemmBatch &batch, WCodec wc) {
 // Examples (us, before -> now): 768 x 3072 x 3072 52 -> 29, 768 x 3072 x 12288
 // 184 -> 102, 1536 x 3072 x 15360 237 -> 176, 768 x 9216 x 3072 58 -> 48.
 // The narrow tile has to win by 4 % (the estimates' error at full rounds).
+// plan_wide_tiles compares wide tiles with each other, by rounds and ratios; these estimates only say whether a narrow
+// one beats its choice, in absolute times. int8_row uses the NF4 table. Checked over the FLUX linears at 28 row counts
+// from 40 to 6144: every launch in narrow tiles beat the wide tile, NF4 by 5 to 49 % (78 launches), int8_row by 14 to
+// 51 % (77; its wide tiles gained 5 to 15 % from the fence in the K loop meanwhile), and no other was slower.
 struct TileCost {
   int mb, cb;
   double f, c, r;
@@ -2308,33 +2312,62 @@ extern "C" int selas_int8_row_linear_batched(const selas_nf4_gemm_problem *probl
                         workspace_bytes, stream);
 }
 
-extern "C" int selas_linear_workspace_bytes(const selas_nf4_gemm_problem *problems, int64_t count, int codec,
-                                            int64_t *bytes) {
-  if (!bytes) return set_error(SELAS_EINVAL, "linear_workspace_bytes: null result pointer");
-  *bytes = 0;
+namespace {
+// The plan of a launch over problems of these shapes: empty (no tiles) where a skinny kernel takes one of them, or none
+// has rows.
+int plan_of(const char *what, const selas_nf4_gemm_problem *problems, int64_t count, int codec, GemmBatch &batch,
+            GemmPlan &plan) {
   if (codec != SELAS_CODEC_NF4 && codec != SELAS_CODEC_INT8_ROW)
-    return set_error(SELAS_EINVAL, "linear_workspace_bytes: unknown codec %d", codec);
+    return set_error(SELAS_EINVAL, "%s: unknown codec %d", what, codec);
   if (count < 0 || count > kGemmMaxProblems)
-    return set_error(SELAS_EINVAL, "linear_workspace_bytes: count %lld outside [0, %d]", (long long)count,
-                     kGemmMaxProblems);
-  if (count > 0 && !problems) return set_error(SELAS_EINVAL, "linear_workspace_bytes: null problems");
-  GemmBatch batch{};
+    return set_error(SELAS_EINVAL, "%s: count %lld outside [0, %d]", what, (long long)count, kGemmMaxProblems);
+  if (count > 0 && !problems) return set_error(SELAS_EINVAL, "%s: null problems", what);
+  batch = GemmBatch{};
   for (int64_t i = 0; i < count; ++i) {
     const selas_nf4_gemm_problem &q = problems[i];
     if (q.M < 0 || q.K <= 0 || q.N <= 0 || q.M > INT32_MAX || q.K > INT32_MAX || q.N > INT32_MAX)
-      return set_error(SELAS_EINVAL, "linear_workspace_bytes: bad shape M=%lld K=%lld N=%lld", (long long)q.M,
-                       (long long)q.K, (long long)q.N);
+      return set_error(SELAS_EINVAL, "%s: bad shape M=%lld K=%lld N=%lld", what, (long long)q.M, (long long)q.K,
+                       (long long)q.N);
     if (q.M == 0) continue;
-    if (q.M <= 32) return ok();  // the skinny kernels, or a batch that runs one by one: no workspace
+    if (q.M <= 32) {
+      batch.count = 0;
+      return ok();
+    }
     GemmProblem &p = batch.p[batch.count++];
     p.M = static_cast<int>(q.M);
     p.K = static_cast<int>(q.K);
     p.N = static_cast<int>(q.N);
   }
-  if (batch.count == 0) return ok();
-  *bytes = plan_gemm(batch, codec == SELAS_CODEC_NF4 ? WCodec::kNF4 : WCodec::kInt8Row).workspace_bytes();
+  if (batch.count) plan = plan_gemm(batch, codec == SELAS_CODEC_NF4 ? WCodec::kNF4 : WCodec::kInt8Row);
   return ok();
 }
+}  // namespace
+
+extern "C" int selas_linear_workspace_bytes(const selas_nf4_gemm_problem *problems, int64_t count, int codec,
+                                            int64_t *bytes) {
+  if (!bytes) return set_error(SELAS_EINVAL, "linear_workspace_bytes: null result pointer");
+  *bytes = 0;
+  GemmBatch batch;
+  GemmPlan plan;
+  if (int e = plan_of("linear_workspace_bytes", problems, count, codec, batch, plan)) return e;
+  if (batch.count) *bytes = plan.workspace_bytes();
+  return ok();
+}
+
+extern "C" int selas_linear_tile(const selas_nf4_gemm_problem *problems, int64_t count, int codec, int64_t *rows,
+                                 int64_t *cols) {
+  if (!rows || !cols) return set_error(SELAS_EINVAL, "linear_tile: null result pointer");
+  *rows = *cols = 0;
+  GemmBatch batch;
+  GemmPlan plan;
+  if (int e = plan_of("linear_tile", problems, count, codec, batch, plan)) return e;
+  if (batch.count) {
+    *rows = 32 * plan.mb;
+    *cols = 128 * plan.cb;
+  }
+  return ok();
+}
+
 
 extern "C" int selas_int8_row_linear(const void *x, int64_t M, int64_t K, int64_t ldx, const int8_t *q,
                                      const float *scale, int64_t N, const void *bias, void *y, int64_t ldy, int dtype,

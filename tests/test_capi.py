@@ -180,6 +180,25 @@ def _ws_query(shapes, codec=_lib.CODEC_NF4):
     return out.value
 
 
+def tile_query(m, n, k, codec=_lib.CODEC_NF4):
+    arr = (_lib.GemmProblem * 1)()
+    arr[0].M, arr[0].K, arr[0].N = m, k, n
+    rows, cols = ctypes.c_int64(-1), ctypes.c_int64(-1)
+    _lib.call("selas_linear_tile", ctypes.addressof(arr), 1, codec, ctypes.byref(rows), ctypes.byref(cols))
+    return rows.value, cols.value
+
+
+def test_tile_shapes():
+    # Narrow tiles where wide ones leave CUs idle, wide ones from a round's fill on; the skinny kernels have none.
+    for codec in (_lib.CODEC_NF4, _lib.CODEC_INT8_ROW):
+        assert tile_query(768, 3072, 3072, codec) == (128, 128) and tile_query(1536, 3072, 15360, codec) == (192, 128)
+        assert tile_query(2048, 3072, 3072, codec) == (256, 128)
+        assert tile_query(4608, 21504, 3072, codec) == (256, 256)
+        assert tile_query(32, 3072, 3072, codec) == tile_query(0, 3072, 3072, codec) == (0, 0)
+    with pytest.raises(ValueError, match="codec"):
+        tile_query(64, 64, 64, codec=7)
+
+
 def test_split_workspace_is_sized_from_shapes_only():
     # The split plan is host logic over (M, K, N) and the CU count (256 on MI355X; the fallback when no GPU
     # answers). 4 x 1536 tokens x 3072 x 15360 (the 512^2 batch-4 linear2): 24 x 12 = 288 tiles of 256 x 256,

@@ -13,11 +13,12 @@ import torch
 
 from oracle import int8_row as oi8
 from oracle import nf4 as onf4
-from selas_amd import codecs
+from selas_amd import _lib, codecs
 from selas_amd.kernels import Kernels
 from selas_amd.linear import int8_row_linear, int8_row_linear_gelu, nf4_linear, nf4_linear_gelu
 
 from .conftest import seeded
+from .test_capi import tile_query
 
 pytestmark = pytest.mark.gpu
 
@@ -35,14 +36,19 @@ def weight(codec, n, k, dev):
     return args, torch.from_numpy(onf4.bf16_to_f32(np.asarray(ref))).view(n, k).double()
 
 
-# On 256 CUs: 128-row tiles at the smallest sizes, with one row past a tile and partial columns (100 rows; 257 x 1000;
-# K of one, two and four blocks: every remainder of the three-block loop); 192 rows (1536 x 3072, 16 x 24 tiles); 256
-# rows x 128 columns (768 x 9216); one row short of and past a tile (767, 769).
-@pytest.mark.parametrize("m,n,k", [(33, 64, 64), (100, 260, 128), (257, 1000, 256), (1536, 3072, 192),
-                                   (767, 9216, 128), (769, 9216, 320), (385, 3072, 3072)])
+# The tile each size runs in on 256 CUs: 128 rows x 128 columns at the smallest, with one row past a tile and partial
+# columns (100 rows; 257 x 1000; K of one, two and four blocks: every remainder of the three-block loop); 192 rows in
+# whole tiles (8 x 24 of them), one row past and one short; 256 rows, one row short of a tile and one past; and the wide
+# tile that follows it at 769 x 9216.
+@pytest.mark.parametrize("m,n,k,tile", [
+    (33, 64, 64, (128, 128)), (100, 260, 128, (128, 128)), (257, 1000, 256, (128, 128)), (385, 3072, 3072, (128, 128)),
+    (1536, 3072, 192, (192, 128)), (1345, 3072, 320, (192, 128)), (575, 9216, 128, (192, 128)),
+    (767, 9216, 128, (256, 128)), (2049, 3072, 320, (256, 128)), (769, 9216, 320, (192, 256))])
 @pytest.mark.parametrize("codec", ["nf4", "int8_row"])
-def test_narrow_tiles(codec, m, n, k):
+def test_narrow_tiles(codec, m, n, k, tile):
     dev = torch.device("cuda")
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        assert tile_query(m, n, k, _lib.CODEC_NF4 if codec == "nf4" else _lib.CODEC_INT8_ROW) == tile
     args, w_ref = weight(codec, n, k, dev)
     lin = nf4_linear if codec == "nf4" else int8_row_linear
     x = torch.randn(m, k, generator=seeded(m)).to(torch.bfloat16).to(dev)
@@ -52,7 +58,7 @@ def test_narrow_tiles(codec, m, n, k):
     ref = x[rows].double().cpu() @ w_ref.t() + b.double().cpu()
     d = y[rows].double().cpu() - ref
     assert d.abs().max() <= 1e-2 * ref.abs().max() and d.norm() <= 4e-3 * ref.norm()
-    big = torch.randn(5000, k, generator=seeded(m + 1)).to(torch.bfloat16).to(dev)  # wider tiles
+    big = torch.randn(5000, k, generator=seeded(m + 1)).to(torch.bfloat16).to(dev)  # elsewhere in a larger launch, most in wider tiles
     big[1111:1111 + m] = x
     assert torch.equal(lin(big, *args, b)[1111:1111 + m], y)
     if n % 256 == 0:  # the GELU columns in the epilogue: the bits of the linear and the GELU segment
