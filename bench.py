@@ -466,21 +466,20 @@ def segment_bytes(kind: str, cfg, l_img: int, l_txt: int, batch: int) -> float:
 
 def bench_attention(dev, steps, warmup):
     """The block attention at 1024^2 (B = 1, 24 heads x 128, L = 4608) and at 512^2 with batch 4 (L = 1536):
-    the fused kernel (its launch alone, and the call with the value transpose) against the reference's
-    SDPA + transpose/reshape (torch's flash backends)."""
+    the fused kernel (its launch alone, output preallocated; neither shape is split over the keys) and the call of
+    the package, against the reference's SDPA + transpose/reshape (torch's flash backends)."""
     from selas_amd import _lib
     from selas_amd import flux as F
-    from selas_amd.attention import attention, transpose_heads
+    from selas_amd.attention import attention
 
     out = {}
     for name, b, l in (("b1_1024", 1, 4608), ("b4_512", 4, 1536)):
         g = torch.Generator(device=dev).manual_seed(6)
         q, k, v = (torch.randn(b, 24, l, 128, generator=g, device=dev).to(torch.bfloat16) for _ in range(3))
-        vt = transpose_heads(v)
         o = torch.empty(b, l, 24 * 128, dtype=torch.bfloat16, device=dev)
 
         def kernel():
-            _lib.call("selas_attention", q.data_ptr(), k.data_ptr(), vt.data_ptr(), b, 24, l, 128, o.data_ptr(),
+            _lib.call("selas_attention_v", q.data_ptr(), k.data_ptr(), v.data_ptr(), b, 24, l, 128, o.data_ptr(),
                       24 * 128, _lib.BF16, _lib.stream(dev))
 
         runs = {"kernel": kernel, "fused_call": lambda: attention(q, k, v), "sdpa": lambda: F.sdpa_attention(q, k, v)}
