@@ -127,8 +127,8 @@ __device__ __forceinline__ uint32_t code_index(float x, const Mids15 &mids) {
 }
 
 // Search table over 64 equal buckets of [-1, 1], each with at most one midpoint: the midpoint's bits with the low four
-// replaced by the number of midpoints in lower buckets (4.0, above every x, where there is no midpoint). One entry per
-// LDS bank: any 64 lanes read it without conflicts.
+// replaced by the number of midpoints in lower buckets (4.0, above every x, where there is no midpoint). 64 words in LDS
+// (1.4 conflict cycles counted per LDS instruction of the kernel, the maximum's shuffles included; HBM-bound with them).
 struct SearchTable {
   uint32_t e[64];
 };
