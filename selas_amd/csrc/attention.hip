@@ -86,7 +86,8 @@ struct AttnSplit {
 // running maximum and the sum.
 constexpr int kPartialFloats = 64 * 64 + 2 * 64;
 
-// VT: the values come as v^T [B*H, 128, Lp] (selas_attention), else as v [B*H, L, 128] (selas_attention_v).
+// VT: the values come as v^T [B*H, 128, Lp] (selas_attention, for callers of the C ABI that have them so), else as v
+// [B*H, L, 128].
 template <int NWV, bool VT, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NWV, 2) void attn_fwd_kernel(const uint16_t *__restrict__ q,
                                                                const uint16_t *__restrict__ k,
