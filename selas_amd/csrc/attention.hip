@@ -497,9 +497,9 @@ double rounds4(int64_t B, int64_t H, int64_t L) {
 // 2688: 92 us), and not for fewer than 40 key tiles (a range's prologue, its partial output and the merge take 8 us).
 // Unsplit / split, us, batch 1 to 4, 24 heads: L 2700 125 / 104, 206 / 188, 308 / 271, 392 / 359; L 3072 138 / 119,
 // 232 / 221, 343 / 334, 446 / 438 (six images 639 / 651, eight 829 / 873); L 5632 406 / 353, 764 / 682; L 6144
-// 448 / 425, 834 / 802. Past the line: L 3328 (56 items over one round) in 3 ranges 151 / 137, 257 / 270, in 2
-// 151 / 144, 257 / 254, 382 / 395; L 4096 (128) 196 / 194, 361 / 379; 32 heads, L 2100 (33 key tiles) 97 / 88 and, batch
-// 4, 304 / 312.
+// 448 / 425, 834 / 802. Past the line: L 3328 (56 items over one round) in 4 ranges 152 / 137, 259 / 266, 381 / 397,
+// 494 / 530, in 2 151 / 144, 257 / 254, 382 / 395; L 3584 (80) in 3 167 / 156, 299 / 301, 425 / 451; L 4096 (128)
+// 196 / 194, 361 / 379; 32 heads, L 2100 (33 key tiles) 97 / 88 and, batch 4, 304 / 312.
 AttnSplit plan_split(int64_t H, int64_t L) {
   AttnSplit split{0, 0, 0, 0, nullptr};
   const int64_t cu = attn_cu_count(), items = H * cdiv(L, 256), tail = items % cu, full = items / cu, tiles = cdiv(L, kKT);
